@@ -1,0 +1,759 @@
+// Device side of the 3D half steps (acoustic fd3d.hip, elastic
+// fd3d_elastic.hip): the z march both share, and the host code that lays out
+// their launches.
+//
+// A block owns a column tile of TX x TY = 512 cells in (x, y), 64 x 8 or
+// 32 x 16, and marches through a chunk of z planes; a thread owns two rows of
+// one column.  The x and y taps of a plane come from LDS (the plane's window
+// with its halo, double buffered: one barrier a plane), the z taps from a
+// register queue of 2*ORDER values per cell.
+//
+// Everything a plane needs is loaded two planes ahead, PML memory variables
+// included, into one of two register sets.  For that to hide the latency no
+// load may be waited for early, and the compiler waits early wherever a value
+// still in flight is moved (so the queue takes its two new values at the top
+// of the next round, two planes after their loads) or wherever a branch makes
+// the number of loads in flight unknown.  So the march has no branches around
+// loads: tiles with strips or shortened stencils in x or y (PXY) and chunks
+// with them in z (PZ) are instantiations of their own, and loads past the end
+// of a chunk use an empty descriptor.
+//
+// What bounds it: HBM on large grids, the march's latency (1.7 us a plane with
+// one block to a SIMD) and the filling of the queue on small ones.  Acoustic,
+// order 4, against 64 x 8 tiles that loaded one plane ahead and the memory
+// variables where they were used, us a velocity + a stress half step:
+// 320 x 300 x 280 333 + 256 -> 238 + 164 (4.5 and 3.9 TB/s algorithmic),
+// 440^3 914 + 677 -> 780 + 477, 160 x 150 x 140 66 + 58 -> 33 + 30,
+// 120 x 110 x 100 42 + 36 -> 19 + 18; order 8, 320 x 300 x 280 519 + 445 ->
+// 264 + 222.
+#pragma once
+#include <algorithm>
+#include <type_traits>
+
+#include "rsg_common.h"
+
+namespace rsg {
+
+constexpr int R3 = 2, B3 = 256;  // rows a thread, threads a block
+
+// Four waves a SIMD up to order 4 (128 VGPRs, no spills); the longer queues of
+// the higher orders need up to 168.
+#define RSG3_BOUNDS(ORDER) __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu((ORDER) <= 4 ? 4 : 3, 8)))
+
+// Raw buffers over the tile's part of an array: every lane either has an
+// offset inside its tile's window of the grid, or kOut, which no descriptor
+// covers: loads return 0 and stores are dropped, so lanes outside the grid
+// need no branches.  A descriptor that is not live covers nothing.
+constexpr unsigned kOut = 0xFFFFFF00u;
+__device__ __forceinline__ Buf tile_buf(const float *f, long off, bool live = true) {
+    return mkbuf(f + off, live ? 0x7FFFFF00u : 0u);
+}
+
+// Byte offset of a plane, hidden from the optimiser: it would otherwise keep
+// one running address per array, load and store (the scalar registers then
+// spill into vector lanes) instead of two scalar adds where one is used.
+__device__ __forceinline__ long opaque(long v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// One derivative term: the field, its two strips (low, high face), and
+// whether it is the forward (1) or backward (0) difference.
+struct Term3 {
+    const float *f;
+    float *lo, *hi;
+    int fw;
+};
+
+// Tile order.  ncx x ncy columns of TX x TY cells; the z planes in three
+// zones (strips or shortened stencils at the low face, neither, the high
+// face), zone i of planes z[i] .. z[i+1]-1 in n[i] chunks of zc planes; ncomp
+// components (blocks that update different arrays of one tile from partly the
+// same inputs).  With xgroups blocks are dealt round-robin to the 8 XCDs (XCD
+// k runs blocks k, k+8, ...) and XCD k marches its own contiguous group of
+// columns cg[k] .. cg[k+1]-1 through the chunks, components fastest, then
+// columns: the blocks an XCD holds at once are neighbours at the same depth,
+// so shared inputs, halos and the lines that tile rows share are fetched into
+// that XCD's L2 once.
+struct Tiles3 {
+    int tx, xgroups, ncx, ncy, zc, ncomp;
+    int z[4], n[3];
+    int cg[9];
+};
+
+struct Pos3 {
+    int x0, y0, zb, ze, comp;
+    bool pz;
+};
+
+template <int TX>
+__device__ __forceinline__ bool tile3_of(const Tiles3 &t, Pos3 &p) {
+    int col, ck, r = blockIdx.x;
+    const int nck = t.n[0] + t.n[1] + t.n[2];
+    if (!t.xgroups) {
+        p.comp = r % t.ncomp;
+        r /= t.ncomp;
+        ck = r / (t.ncx * t.ncy);
+        col = r - ck * (t.ncx * t.ncy);
+    } else {
+        const int k = r % 8, ncol = t.cg[k + 1] - t.cg[k];
+        r /= 8;
+        p.comp = r % t.ncomp;
+        r /= t.ncomp;
+        if (ncol <= 0 || r >= ncol * nck) return false;
+        ck = r / ncol;
+        col = t.cg[k] + (r - ck * ncol);
+    }
+    const int cy = col / t.ncx;
+    p.x0 = (col - cy * t.ncx) * TX;
+    p.y0 = cy * (R3 * B3 / TX);
+    int zone = 0;
+    if (ck >= t.n[0]) {
+        ck -= t.n[0];
+        zone = 1;
+        if (ck >= t.n[1]) {
+            ck -= t.n[1];
+            zone = 2;
+        }
+    }
+    p.zb = t.z[zone] + ck * t.zc;
+    p.ze = min(p.zb + t.zc, t.z[zone + 1]);
+    p.pz = zone != 1;
+    return p.zb < p.ze;
+}
+
+// Grid, step and stencil description every 3D kernel takes.
+struct G3 {
+    int nx, ny, nz, lpml, fs, order;
+    float dt, inv[3];
+    const float *tab;
+    float c[3][8];   // the stencil's coefficients over the step, per axis
+    float cz[9][8];  // z: of every order (0 past it), for the planes at the ends
+    Tiles3 t;
+};
+
+// Does the tile hold cells of x or y strips, or whose x or y stencils the
+// array's ends shorten, or cells outside the grid?
+template <int TX>
+__device__ __forceinline__ bool tile_pxy(const G3 &g, const Pos3 &p) {
+    const int m = max(g.lpml, g.order);
+    return p.x0 < m || p.x0 + TX > g.nx - m || p.y0 < m || p.y0 + R3 * B3 / TX > g.ny - m;
+}
+
+// z-derivative from a queue q[j] = f(z + off + j): both the forward
+// (off = 1-H) and the backward (off = -H) staggered forms reduce to
+// sum_io c_io (q[H+io] - q[H-1-io]).  The queue holds two more values than a
+// plane takes: odd planes of a chunk (S = 1) read it one further, and it
+// shifts once every two planes.
+template <int H, int S>
+__device__ __forceinline__ float dq(const float (&q)[2 * H + 2], const float *c) {
+    float acc = c[0] * (q[S + H] - q[S + H - 1]);
+#pragma unroll
+    for (int io = 1; io < H; io++) acc += c[io] * (q[S + H + io] - q[S + H - 1 - io]);
+    return acc;
+}
+template <int N>
+__device__ __forceinline__ void shift2(float (&q)[R3][N], const float (&qn)[2][R3]) {
+#pragma unroll
+    for (int r = 0; r < R3; r++) {
+#pragma unroll
+        for (int j = 0; j < N - 2; j++) q[r][j] = q[r][j + 2];
+        q[r][N - 2] = qn[0][r];
+        q[r][N - 1] = qn[1][r];
+    }
+}
+
+// The forward difference of a cell whose stencil the array's end shortens to
+// order k, coefficients from a table in LDS (a global load here would wait
+// for every load in flight).
+__device__ __forceinline__ float dfw_edge(const float *s, int st, int k, float invd, const float *ce) {
+    const float *c = ce + cind(k);
+    float acc = 0.f;
+#pragma unroll 1
+    for (int io = 0; io < k; io++) acc += c[io] * (s[(io + 1) * st] - s[-io * st]);
+    return acc * invd;
+}
+
+// Window of one plane, TY + 2*HY rows of TX + 2*HX: each thread's element
+// list (offsets from the window's corner, kOut outside the grid) is fixed for
+// the whole march; fetch loads into registers, store writes them to LDS.
+template <int TX, int HX, int HY>
+struct Win3 {
+    static constexpr int LD = TX + 2 * HX, N = LD * (R3 * B3 / TX + 2 * HY), K = (N + B3 - 1) / B3;
+    unsigned off[K];
+    __device__ __forceinline__ void init(int nx, int ny, int x0, int y0) {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int i = (int)threadIdx.x + k * B3, r = i / LD, c = i - r * LD;
+            const int y = y0 - HY + r, x = x0 - HX + c;
+            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? (unsigned)((r * nx + c) * 4) : kOut;
+        }
+    }
+    // f at plane offset `at` (of the tile's first cell)
+    __device__ __forceinline__ void fetch(float (&v)[K], const float *f, long at, int nx, bool live) const {
+        const Buf b = tile_buf(f, at - (long)HY * nx - HX, live);
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k] = b.ld(off[k], 0);
+    }
+    __device__ __forceinline__ void store(const float (&v)[K], float *lds) const {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (N % B3 == 0 || (int)threadIdx.x + k * B3 < N) lds[threadIdx.x + k * B3] = v[k];
+    }
+};
+
+// A lane's cell against the strips of the x or y axis: its memory variable on
+// the chunk's first plane (a lane outside the strips points at some cell of
+// theirs, so that its load needs no branch) and its profile values.
+struct Face3 {
+    float *psi;
+    float A, B, C;
+    bool in;
+    // i: the cell on the axis (any, where not ok); off(j): index of strip cell j
+    template <class F>
+    __device__ __forceinline__ void init(int i, int n, int L, bool ok, float *lo, float *hi, F &&off, const float *tab,
+                                         int stag) {
+        const bool h = i >= n - L;
+        in = ok && (i < L || h);
+        const int j = !in ? 0 : (h ? i - (n - L) : i), s = (h ? T_RBB : 0) + stag * T_STAG;
+        psi = (h ? hi : lo) + off(j);
+        A = tab[(s + T_A) * L + j];
+        B = tab[(s + T_B) * L + j];
+        C = tab[(s + T_C) * L + j];
+    }
+};
+
+// A thread's cells: column x, rows y .. y+R3-1, and their offsets in the
+// tile's part of a plane (kOut outside the grid).
+template <int TX>
+struct Lane3 {
+    int tx, ty, x, y;
+    unsigned oc[R3];
+    bool ok[R3];
+    long t0;  // the tile's first cell in a plane
+    __device__ __forceinline__ Lane3(const G3 &g, const Pos3 &p) {
+        tx = threadIdx.x % TX;
+        ty = threadIdx.x / TX;
+        x = p.x0 + tx;
+        y = p.y0 + ty * R3;
+#pragma unroll
+        for (int r = 0; r < R3; r++) {
+            ok[r] = x < g.nx && y + r < g.ny;
+            oc[r] = ok[r] ? (unsigned)(((ty * R3 + r) * g.nx + tx) * 4) : kOut;
+        }
+        t0 = (long)p.y0 * g.nx + p.x0;
+    }
+    __device__ __forceinline__ long at(const G3 &g, int z) const { return opaque(z * ((long)g.nx * g.ny) + t0); }
+    __device__ __forceinline__ void ld(const float *f, long o, float (&v)[R3], bool live = true) const {
+        const Buf b = tile_buf(f, o, live);
+#pragma unroll
+        for (int r = 0; r < R3; r++) v[r] = b.ld(oc[r], 0);
+    }
+    __device__ __forceinline__ void st(float *f, long o, const float (&v)[R3]) const {
+        const Buf b = tile_buf(f, o);
+#pragma unroll
+        for (int r = 0; r < R3; r++) b.st(v[r], oc[r], 0);
+    }
+    // f at plane z of the own cells (0 outside the grid, or where not live)
+    __device__ __forceinline__ void queue(const float *f, int z, const G3 &g, float (&v)[R3], bool live = true) const {
+        const bool in = live && z >= 0 && z < g.nz;
+        ld(f, at(g, in ? z : 0), v, in);
+    }
+    // the queue before its first shift: values of planes z .. in q[2 ..] and qn
+    template <int N>
+    __device__ __forceinline__ void fill(const float *f, int z, const G3 &g, float (&q)[R3][N], float (&qn)[2][R3]) const {
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            float v[R3];
+            queue(f, z + j, g, v);
+#pragma unroll
+            for (int r = 0; r < R3; r++) (j < N - 2 ? q[r][j + 2] : qn[j - (N - 2)][r]) = v[r];
+        }
+#pragma unroll
+        for (int r = 0; r < R3; r++) q[r][0] = q[r][1] = 0.f;
+    }
+};
+
+// The x and y strips of a PXY tile.
+template <int TX>
+struct Sides3 {
+    Face3 x, y[R3];
+    int xr;              // rows apart in an x strip (0: the second row is outside the grid)
+    long xstep, ystep;   // planes apart
+    int kx, ky[R3];      // stencil orders
+    __device__ __forceinline__ void init(const G3 &g, const Pos3 &p, const Lane3<TX> &ln, const Term3 &tx, const Term3 &ty) {
+        const int nx = g.nx, ny = g.ny, L = g.lpml, H = g.order;
+        xstep = (long)ny * L;
+        ystep = (long)L * nx;
+        const int xc = min(ln.x, nx - 1), yc = min(ln.y, ny - 1);
+        xr = ln.ok[1] ? L : 0;
+        if (tx.f)
+            x.init(xc, nx, L, ln.ok[0], tx.lo, tx.hi, [&](int j) { return p.zb * xstep + (long)yc * L + j; }, g.tab, tx.fw);
+        kx = tx.fw ? kfw(ln.x, nx, H) : kbw(ln.x, nx, H);
+#pragma unroll
+        for (int r = 0; r < R3; r++) {
+            if (ty.f)
+                y[r].init(min(ln.y + r, ny - 1), ny, L, ln.ok[r], ty.lo, ty.hi,
+                          [&](int j) { return p.zb * ystep + (long)j * nx + xc; }, g.tab, ty.fw);
+            ky[r] = ty.fw ? kfw(ln.y + r, ny, H) : kbw(ln.y + r, ny, H);
+        }
+    }
+    // memory variables k planes on
+    __device__ __forceinline__ void load_x(float (&v)[R3], int k) const {
+#pragma unroll
+        for (int r = 0; r < R3; r++) v[r] = x.psi[k * xstep + r * xr];
+    }
+    __device__ __forceinline__ void load_y(float (&v)[R3], int k) const {
+#pragma unroll
+        for (int r = 0; r < R3; r++) v[r] = y[r].psi[k * ystep];
+    }
+    __device__ __forceinline__ bool in_x(const Lane3<TX> &ln, int r) const { return x.in && ln.ok[r]; }
+    __device__ __forceinline__ void next() {
+        x.psi += 2 * xstep;
+#pragma unroll
+        for (int r = 0; r < R3; r++) y[r].psi += 2 * ystep;
+    }
+};
+
+// The z strips of a plane: memory variables of the own cells and the plane's
+// profile values.  A plane between the strips (a PZ chunk of a grid whose
+// strips are thinner than the stencil) loads nothing and has in = false.
+struct ZPml {
+    float A, B, C, v[R3];
+    __device__ __forceinline__ static bool inside(const G3 &g, int z, bool &h, int &j) {
+        h = z >= g.nz - g.lpml;
+        j = h ? z - (g.nz - g.lpml) : z;
+        return z < g.lpml || h;
+    }
+    template <int TX>
+    __device__ __forceinline__ void load(const G3 &g, const Term3 &t, int z, const Lane3<TX> &ln, bool live) {
+        bool h;
+        int j;
+        const bool in = inside(g, z, h, j) && live;
+        const float *tb = g.tab + ((h ? T_RBB : 0) + t.fw * T_STAG) * g.lpml + (in ? j : 0);
+        A = tb[T_A * g.lpml];
+        B = tb[T_B * g.lpml];
+        C = tb[T_C * g.lpml];
+        ln.ld(h ? t.hi : t.lo, opaque((in ? j : 0) * ((long)g.nx * g.ny) + ln.t0), v, in);
+    }
+    template <int TX>
+    __device__ __forceinline__ void store(const G3 &g, const Term3 &t, int z, const Lane3<TX> &ln) const {
+        bool h;
+        int j;
+        const bool in = inside(g, z, h, j);
+        const Buf b = tile_buf(h ? t.hi : t.lo, opaque((in ? j : 0) * ((long)g.nx * g.ny) + ln.t0), in);
+#pragma unroll
+        for (int r = 0; r < R3; r++) b.st(v[r], ln.oc[r], 0);
+    }
+};
+
+// psi = B psi + A d; F -= m (psi + C d) for a cell in the strip.
+__device__ __forceinline__ void strip3(float &F, float m, float d, bool in, float C, float psi) {
+    F = in ? F - m * (psi + C * d) : F;
+}
+
+// Two planes a round: body(S, z) for the even (S = 0) and odd (S = 1) planes
+// of [zb, ze), top(z) before each pair, next() after it.
+template <class T, class B, class N>
+__device__ __forceinline__ void march3(int zb, int ze, T &&top, B &&body, N &&next) {
+    constexpr std::integral_constant<int, 0> S0;
+    constexpr std::integral_constant<int, 1> S1;
+#pragma unroll 1
+    for (int z = zb;;) {
+        top(z);
+        body(S0, z);
+        if (z + 1 >= ze) break;
+        body(S1, z + 1);
+        next();
+        z += 2;
+        if (z >= ze) break;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// F_i += dt M_i (Dx fx + Dy fy + Dz fz), each term with its CFS-PML memory
+// variable: the acoustic stress step, an elastic velocity component, the
+// elastic normal stresses (NOUT 3: moduli L + 2 mu of the component's own
+// axis, L of the others; UNIT: F_i += dt of its own term) and, with one term
+// left out, an elastic shear stress.
+// ---------------------------------------------------------------------------
+
+struct Comp3 {
+    Term3 t[3];         // x, y, z
+    float *F[3];        // NOUT of them
+    const float *M[2];  // the modulus (NOUT 1), or L, L + 2 mu
+};
+
+template <int TX, int ORDER, bool HX, bool HY, bool HZ, int NOUT, bool UNIT>
+struct Div3 {
+    static constexpr int H = ORDER, NM = UNIT ? 0 : (NOUT == 3 ? 2 : 1);
+    using WX = Win3<TX, H, 0>;
+    using WY = Win3<TX, 0, H>;
+    // floats of LDS: two buffers of both windows, and the edge coefficients
+    static constexpr int LX = HX ? WX::N : 0, LY = HY ? WY::N : 0, LDS = 2 * (LX + LY) + 36;
+
+    template <bool PXY, bool PZ>
+    static __device__ __forceinline__ void march(const G3 &g, const Comp3 &c, const Pos3 &p, float *lds) {
+        const int fx = c.t[0].fw, fy = c.t[1].fw, fz = c.t[2].fw, nx = g.nx;
+        const Lane3<TX> ln(g, p);
+        float *const ce = lds + 2 * (LX + LY);
+        WX wx;
+        WY wy;
+        if (HX) wx.init(nx, g.ny, p.x0, p.y0);
+        if (HY) wy.init(nx, g.ny, p.x0, p.y0);
+        Sides3<TX> sd;
+        if (PXY) {
+            sd.init(g, p, ln, c.t[0], c.t[1]);
+            if (threadIdx.x < 36) ce[threadIdx.x] = kCoefC[threadIdx.x];
+        }
+        // two sets of a plane's values (even and odd planes of the chunk)
+        float F[2][NOUT][R3], M[2][NM ? NM : 1][R3], sx[2][R3], sy[2][R3], q[R3][2 * H + 2], qn[2][R3];
+        float wvx[2][WX::K], wvy[2][WY::K];
+        ZPml zp[2];
+        auto window = [&](auto S, int z) {
+            constexpr int s = decltype(S)::value;
+            const bool live = z < p.ze;
+            const long at = ln.at(g, live ? z : 0);
+            if (HX) wx.fetch(wvx[s], c.t[0].f, at, nx, live);
+            if (HY) wy.fetch(wvy[s], c.t[1].f, at, nx, live);
+        };
+        // the own cells and memory variables of plane z, k planes from the
+        // strips' current one
+        auto own = [&](auto S, int z, int k) {
+            constexpr int s = decltype(S)::value;
+            const bool live = z < p.ze;
+            const long at = ln.at(g, live ? z : 0);
+#pragma unroll
+            for (int i = 0; i < NOUT; i++) ln.ld(c.F[i], at, F[s][i], live);
+#pragma unroll
+            for (int i = 0; i < NM; i++) ln.ld(c.M[i], at, M[s][i], live);
+            if (PXY && HX) sd.load_x(sx[s], live ? k : 0);
+            if (PXY && HY) sd.load_y(sy[s], live ? k : 0);
+            if (PZ && HZ) zp[s].load(g, c.t[2], z, ln, live);
+        };
+        constexpr std::integral_constant<int, 0> S0;
+        constexpr std::integral_constant<int, 1> S1;
+        if (HZ) ln.fill(c.t[2].f, p.zb + fz - H, g, q, qn);
+        window(S0, p.zb);
+        own(S0, p.zb, 0);
+        window(S1, p.zb + 1);
+        own(S1, p.zb + 1, 1);
+        auto top = [&](int z) {
+            if (HZ) {
+                shift2(q, qn);
+                ln.queue(c.t[2].f, z + 2 + fz + H, g, qn[0], z + 2 < p.ze);
+                ln.queue(c.t[2].f, z + 3 + fz + H, g, qn[1], z + 3 < p.ze);
+            }
+        };
+        auto body = [&](auto S, int z) {
+            constexpr int s = decltype(S)::value;
+            float *const bx = lds + s * (LX + LY), *const by = bx + LX;
+            if (HX) wx.store(wvx[s], bx);
+            if (HY) wy.store(wvy[s], by);
+            __syncthreads();
+            window(S, z + 2);
+            float cz[H];
+#pragma unroll
+            for (int i = 0; i < H; i++) cz[i] = PZ ? g.cz[fz ? kfw(z, g.nz, H) : kbw(z, g.nz, H)][i] : g.c[2][i];
+            bool zh;
+            int zj;
+            const bool zin = PZ && ZPml::inside(g, z, zh, zj);
+#pragma unroll
+            for (int r = 0; r < R3; r++) {
+                const int yl = ln.ty * R3 + r;
+                auto m = [&](int a, int i) { return UNIT ? g.dt : g.dt * M[s][NOUT == 3 && i == a ? NM - 1 : 0][r]; };
+                auto plain = [&](int a, float d) {
+#pragma unroll
+                    for (int i = 0; i < NOUT; i++)
+                        if (!(NOUT == 3 && UNIT && i != a)) F[s][i][r] += m(a, i) * d;
+                };
+                auto strip = [&](int a, float d, bool in, float C, float psi) {
+#pragma unroll
+                    for (int i = 0; i < NOUT; i++)
+                        if (!(NOUT == 3 && UNIT && i != a)) strip3(F[s][i][r], m(a, i), d, in, C, psi);
+                };
+                if (HX) {
+                    // the backward difference is the forward one a cell before
+                    const float *w = bx + yl * WX::LD + ln.tx + H - 1 + fx;
+                    float d = dfw<ORDER>(w, 1, g.c[0]);
+                    if (PXY && sd.kx != H) d = dfw_edge(w, 1, sd.kx, g.inv[0], ce);
+                    plain(0, d);
+                    if (PXY) {
+                        sx[s][r] = sd.x.B * sx[s][r] + sd.x.A * d;
+                        strip(0, d, sd.in_x(ln, r), sd.x.C, sx[s][r]);
+                    }
+                }
+                if (HY) {
+                    const float *w = by + (yl + H - 1 + fy) * WY::LD + ln.tx;
+                    float d = dfw<ORDER>(w, WY::LD, g.c[1]);
+                    if (PXY && sd.ky[r] != H) d = dfw_edge(w, WY::LD, sd.ky[r], g.inv[1], ce);
+                    plain(1, d);
+                    if (PXY) {
+                        sy[s][r] = sd.y[r].B * sy[s][r] + sd.y[r].A * d;
+                        strip(1, d, sd.y[r].in, sd.y[r].C, sy[s][r]);
+                    }
+                }
+                if (HZ) {
+                    const float d = dq<H, s>(q[r], cz);
+                    plain(2, d);
+                    if (PZ) {
+                        zp[s].v[r] = zp[s].B * zp[s].v[r] + zp[s].A * d;
+                        strip(2, d, zin, zp[s].C, zp[s].v[r]);
+                    }
+                }
+                // free surface: the plane lpml lies in no z strip, so zeroing
+                // after the strips is the reference's zeroing before them
+                if (NOUT == 3 && g.fs && z == g.lpml) F[s][NOUT - 1][r] = 0.f;
+            }
+            const long at = ln.at(g, z);
+#pragma unroll
+            for (int i = 0; i < NOUT; i++) ln.st(c.F[i], at, F[s][i]);
+            if (PZ && HZ) zp[s].store(g, c.t[2], z, ln);
+            if (PXY)
+#pragma unroll
+                for (int r = 0; r < R3; r++) {
+                    if (HX && sd.in_x(ln, r)) sd.x.psi[s * sd.xstep + r * sd.xr] = sx[s][r];
+                    if (HY && sd.y[r].in) sd.y[r].psi[s * sd.ystep] = sy[s][r];
+                }
+            own(S, z + 2, s + 2);
+        };
+        march3(p.zb, p.ze, top, body, [&]() {
+            if (PXY) sd.next();
+        });
+    }
+
+    static __device__ __forceinline__ void run(const G3 &g, const Comp3 &c, const Pos3 &p, float *lds) {
+        if (tile_pxy<TX>(g, p)) {
+            if (p.pz && HZ)
+                march<true, true>(g, c, p, lds);
+            else
+                march<true, false>(g, c, p, lds);
+        } else {
+            if (p.pz && HZ)
+                march<false, true>(g, c, p, lds);
+            else
+                march<false, false>(g, c, p, lds);
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Acoustic velocity: V_a += dt R_a D+_a P, each with its memory variable.  One
+// field in, three out: P's window carries both halos.
+// ---------------------------------------------------------------------------
+
+struct Grad3Args {
+    Term3 t[3];  // f: P, fw: 1
+    float *V[3];
+    const float *R[3];
+};
+
+template <int TX, int ORDER>
+struct Grad3 {
+    static constexpr int H = ORDER;
+    using W = Win3<TX, H, H>;
+    static constexpr int LDS = 2 * W::N + 36;
+
+    template <bool PXY, bool PZ>
+    static __device__ __forceinline__ void march(const G3 &g, const Grad3Args &c, const Pos3 &p, float *lds) {
+        const float *P = c.t[0].f;
+        const Lane3<TX> ln(g, p);
+        const int nx = g.nx;
+        float *const ce = lds + 2 * W::N;
+        W w;
+        w.init(nx, g.ny, p.x0, p.y0);
+        Sides3<TX> sd;
+        if (PXY) {
+            sd.init(g, p, ln, c.t[0], c.t[1]);
+            if (threadIdx.x < 36) ce[threadIdx.x] = kCoefC[threadIdx.x];
+        }
+        float V[2][3][R3], R[2][3][R3], sx[2][R3], sy[2][R3], wv[2][W::K], q[R3][2 * H + 2], qn[2][R3];
+        ZPml zp[2];
+        auto window = [&](auto S, int z) {
+            const bool live = z < p.ze;
+            w.fetch(wv[decltype(S)::value], P, ln.at(g, live ? z : 0), nx, live);
+        };
+        auto own = [&](auto S, int z, int k) {
+            constexpr int s = decltype(S)::value;
+            const bool live = z < p.ze;
+            const long at = ln.at(g, live ? z : 0);
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                ln.ld(c.V[a], at, V[s][a], live);
+                ln.ld(c.R[a], at, R[s][a], live);
+            }
+            if (PXY) {
+                sd.load_x(sx[s], live ? k : 0);
+                sd.load_y(sy[s], live ? k : 0);
+            }
+            if (PZ) zp[s].load(g, c.t[2], z, ln, live);
+        };
+        constexpr std::integral_constant<int, 0> S0;
+        constexpr std::integral_constant<int, 1> S1;
+        ln.fill(P, p.zb + 1 - H, g, q, qn);
+        window(S0, p.zb);
+        own(S0, p.zb, 0);
+        window(S1, p.zb + 1);
+        own(S1, p.zb + 1, 1);
+        auto top = [&](int z) {
+            shift2(q, qn);
+            ln.queue(P, z + 3 + H, g, qn[0], z + 2 < p.ze);
+            ln.queue(P, z + 4 + H, g, qn[1], z + 3 < p.ze);
+        };
+        auto body = [&](auto S, int z) {
+            constexpr int s = decltype(S)::value;
+            float *const b = lds + s * W::N;
+            w.store(wv[s], b);
+            __syncthreads();
+            window(S, z + 2);
+            float cz[H];
+#pragma unroll
+            for (int i = 0; i < H; i++) cz[i] = PZ ? g.cz[kfw(z, g.nz, H)][i] : g.c[2][i];
+            bool zh;
+            int zj;
+            const bool zin = PZ && ZPml::inside(g, z, zh, zj);
+#pragma unroll
+            for (int r = 0; r < R3; r++) {
+                const float *t = b + (ln.ty * R3 + r + H) * W::LD + ln.tx + H;
+                float m = g.dt * R[s][0][r], d = dfw<ORDER>(t, 1, g.c[0]);
+                if (PXY && sd.kx != H) d = dfw_edge(t, 1, sd.kx, g.inv[0], ce);
+                V[s][0][r] += m * d;
+                if (PXY) {
+                    sx[s][r] = sd.x.B * sx[s][r] + sd.x.A * d;
+                    strip3(V[s][0][r], m, d, sd.in_x(ln, r), sd.x.C, sx[s][r]);
+                }
+                m = g.dt * R[s][1][r];
+                d = dfw<ORDER>(t, W::LD, g.c[1]);
+                if (PXY && sd.ky[r] != H) d = dfw_edge(t, W::LD, sd.ky[r], g.inv[1], ce);
+                V[s][1][r] += m * d;
+                if (PXY) {
+                    sy[s][r] = sd.y[r].B * sy[s][r] + sd.y[r].A * d;
+                    strip3(V[s][1][r], m, d, sd.y[r].in, sd.y[r].C, sy[s][r]);
+                }
+                m = g.dt * R[s][2][r];
+                d = dq<H, s>(q[r], cz);
+                V[s][2][r] += m * d;
+                if (PZ) {
+                    zp[s].v[r] = zp[s].B * zp[s].v[r] + zp[s].A * d;
+                    strip3(V[s][2][r], m, d, zin, zp[s].C, zp[s].v[r]);
+                }
+            }
+            const long at = ln.at(g, z);
+#pragma unroll
+            for (int a = 0; a < 3; a++) ln.st(c.V[a], at, V[s][a]);
+            if (PZ) zp[s].store(g, c.t[2], z, ln);
+            if (PXY)
+#pragma unroll
+                for (int r = 0; r < R3; r++) {
+                    if (sd.in_x(ln, r)) sd.x.psi[s * sd.xstep + r * sd.xr] = sx[s][r];
+                    if (sd.y[r].in) sd.y[r].psi[s * sd.ystep] = sy[s][r];
+                }
+            own(S, z + 2, s + 2);
+        };
+        march3(p.zb, p.ze, top, body, [&]() {
+            if (PXY) sd.next();
+        });
+    }
+
+    static __device__ __forceinline__ void run(const G3 &g, const Grad3Args &c, const Pos3 &p, float *lds) {
+        if (tile_pxy<TX>(g, p)) {
+            if (p.pz)
+                march<true, true>(g, c, p, lds);
+            else
+                march<true, false>(g, c, p, lds);
+        } else {
+            if (p.pz)
+                march<false, true>(g, c, p, lds);
+            else
+                march<false, false>(g, c, p, lds);
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Host side
+// ---------------------------------------------------------------------------
+
+static G3 make_g3(const rsg_grid *g, const float *tab, int order) {
+    G3 k{};
+    k.nx = g->nx;
+    k.ny = g->ny;
+    k.nz = g->nz;
+    k.lpml = g->lpml;
+    k.fs = g->fs;
+    k.order = order;
+    k.dt = g->dt;
+    const float d[3] = {g->dx, g->dy, g->dz};
+    for (int a = 0; a < 3; a++) {
+        k.inv[a] = 1.0f / d[a];
+        const Coefs cf = scaled_coefs(d[a]);
+        for (int i = 0; i < order; i++) k.c[a][i] = cf.c[cind(order) + i];
+        if (a == 2)
+            for (int o = 1; o <= order; o++)
+                for (int i = 0; i < o; i++) k.cz[o][i] = cf.c[cind(o) + i];
+    }
+    k.tab = tab;
+    return k;
+}
+
+// Launch grid of ncomp components, and the tile order.
+static unsigned layout3(G3 &k, int ncomp) {
+    Tiles3 &t = k.t;
+    // Rows of 64 touch fewer partly used cache lines (440^3, order 4: 778 + 474
+    // us a step against 873 + 514 with 32), unless they waste much more of a
+    // narrow grid's last tile (160 x 150 x 140: 36 + 33 us against 33 + 29).
+    const int w64 = (k.nx + 63) / 64 * 64, w32 = (k.nx + 31) / 32 * 32;
+    t.tx = 10 * w64 <= 11 * w32 ? 64 : 32;
+    const int ty = R3 * B3 / t.tx;
+    t.ncx = (k.nx + t.tx - 1) / t.tx;
+    t.ncy = (k.ny + ty - 1) / ty;
+    t.ncomp = ncomp;
+    const int m = std::max(k.lpml, k.order), lo = std::min(m, k.nz), hi = std::max(lo, k.nz - m);
+    t.z[0] = 0;
+    t.z[1] = lo;
+    t.z[2] = hi;
+    t.z[3] = k.nz;
+    const long cols = (long)t.ncx * t.ncy * ncomp;
+    auto split = [&](int zc) {
+        t.zc = zc;
+        for (int i = 0; i < 3; i++) t.n[i] = (t.z[i + 1] - t.z[i] + zc - 1) / zc;
+        return t.n[0] + t.n[1] + t.n[2];
+    };
+    int zc = tuning().zc3d;
+    if (zc <= 0) {
+        // Short chunks give many blocks, long ones amortise the queue's
+        // filling: 8 planes where that gives four rounds of blocks (320 x 300 x
+        // 280: 230 + 155 us a step with 8, 235 + 158 with 12, 250 + 169 with
+        // 24), else 4 (120 x 110 x 100: 19 + 18 us with 4, 21 + 22 with 8).
+        zc = cols * split(8) >= 4096 ? 8 : 4;
+    }
+    const int nck = split(zc), ncol = t.ncx * t.ncy;
+    t.xgroups = tuning().xcd3d ? 1 : 0;
+    if (!t.xgroups) return (unsigned)((long)ncol * nck * ncomp);
+    int most = 0;
+    for (int x = 0; x <= 8; x++) {
+        t.cg[x] = (int)((long)ncol * x / 8);
+        if (x) most = std::max(most, t.cg[x] - t.cg[x - 1]);
+    }
+    return (unsigned)(8L * most * nck * ncomp);
+}
+
+#define RSG3_ORDER_CASES(LAUNCH, X, ORDER) \
+    switch (ORDER) {                        \
+    case 1: LAUNCH(X, 1); break;            \
+    case 2: LAUNCH(X, 2); break;            \
+    case 3: LAUNCH(X, 3); break;            \
+    case 4: LAUNCH(X, 4); break;            \
+    case 5: LAUNCH(X, 5); break;            \
+    case 6: LAUNCH(X, 6); break;            \
+    case 7: LAUNCH(X, 7); break;            \
+    default: LAUNCH(X, 8); break;           \
+    }
+#define RSG3_DISPATCH(K, LAUNCH)                    \
+    if ((K).t.tx == 64) {                           \
+        RSG3_ORDER_CASES(LAUNCH, 64, (K).order)     \
+    } else {                                        \
+        RSG3_ORDER_CASES(LAUNCH, 32, (K).order)     \
+    }
+
+}  // namespace rsg
