@@ -6,7 +6,7 @@
 namespace rsg {
 
 template <int TX, int ORDER>
-__global__ RSG3_BOUNDS(ORDER) void a3d_velocity_kernel(const G3 g, const Grad3Args a) {
+__global__ RSG3_BOUNDS void a3d_velocity_kernel(const G3 g, const Grad3Args a) {
     using K = Grad3<TX, ORDER>;
     __shared__ float lds[K::LDS];
     Pos3 p;
@@ -14,7 +14,7 @@ __global__ RSG3_BOUNDS(ORDER) void a3d_velocity_kernel(const G3 g, const Grad3Ar
 }
 
 template <int TX, int ORDER>
-__global__ RSG3_BOUNDS(ORDER) void a3d_stress_kernel(const G3 g, const Comp3 c) {
+__global__ RSG3_BOUNDS void a3d_stress_kernel(const G3 g, const Comp3 c) {
     using K = Div3<TX, ORDER, true, true, true, 1, false>;
     __shared__ float lds[K::LDS];
     Pos3 p;

@@ -5,24 +5,25 @@
 // injection and receiver gathers, and ModelElastic3D::staggerModels on the
 // host (bit-exact, model.cpp:3371-3473).
 //
-// Kernels: one thread per cell, blocks of 64 (x) by 4 (y) cells, one z plane
-// per block row of the grid.  Every derivative reads its stencil straight
-// from HBM: the x stencil is coalesced within the wave, the y and z stencils
-// hit the L2 lines the neighbouring blocks and planes brought in.  Cells whose
-// stencils are at the full order take the compile-time stencil with the
-// coefficients pre-divided by the step; edge cells take the reference's
-// reduced orders.  Each derivative term is applied as the reference applies
-// it: F += dt M d, then in a strip psi = B psi + A d, F -= dt M (psi + C d).
-// Results agree with the reference to rounding (contraction is on here).
+// Kernels: the z march of rsg_fd3d.h, one block per tile, chunk and component:
+// the three velocities (three derivatives into one field each), the normal
+// stresses together (three derivatives into three fields) and each shear
+// stress.  A component needs one queue of z taps, where a block that updated
+// all of them would need three (96 registers a cell pair at order 8); the
+// blocks of one tile run side by side on one XCD, so the fields two components
+// read come from its L2.  Each derivative term is applied as the reference
+// applies it: F += dt M d, then in a strip psi = B psi + A d,
+// F -= dt M (psi + C d).  Results agree with the reference to rounding
+// (contraction is on here).
 //
 // The adjoint-state steps of FwiElastic3D (backwardstepVelocity / Stress,
 // waves.cpp:3260-4103) share the kernels: the velocity step differentiates
 // the moduli-weighted stresses (L2M Sxx + L Syy + L Szz, M_xy Sxy, ...),
-// formed at each stencil point where the reference first fills its wrk
-// array, and the stress step adds bare velocity derivatives.
-#include <vector>
-
-#include "rsg_common.h"
+// written to a workspace first as the reference fills its wrk array, and the
+// stress step adds bare velocity derivatives.  Without a workspace
+// (rsg_e3d_backward_velocity) one thread per cell forms the products at each
+// stencil point, reading them through the caches.
+#include "rsg_e3d.h"
 #include "rsg_fwi.h"
 
 namespace rsg {
@@ -81,17 +82,6 @@ __device__ __forceinline__ bool cell_of(const K3E &k, Cell &cl) {
     return true;
 }
 
-// Derivative of f along axis a at the cell: forward (D+) or backward (D-).
-template <int ORDER, bool FWD>
-__device__ __forceinline__ float deriv(const K3E &k, const Cell &cl, const float *f, int a) {
-    const int n = a == 0 ? k.nx : (a == 1 ? k.ny : k.nz);
-    const int kk = FWD ? kfw(cl.c[a], n, ORDER) : kbw(cl.c[a], n, ORDER);
-    const float *s = f + cl.p;
-    const int st = (int)cl.st[a];
-    if (kk == ORDER) return FWD ? dfw<ORDER>(s, st, k.c[a].c + cind(ORDER)) : dbw<ORDER>(s, st, k.c[a].c + cind(ORDER));
-    return FWD ? dfw_k(s, st, kk, k.invd[a]) : dbw_k(s, st, kk, k.invd[a]);
-}
-
 // Moduli-weighted sum of N stress fields at a cell: the wrk array of
 // backwardstepVelocity, m[0] f[0] + m[1] f[1] + m[2] f[2] in that order.
 template <int N>
@@ -105,7 +95,8 @@ struct Mix {
     }
 };
 
-// deriv for a field given by a functor of the cell index.
+// Derivative along axis a, forward (D+) or backward (D-), of a field given by a
+// functor of the cell index.
 template <int ORDER, bool FWD, class G>
 __device__ __forceinline__ float derivm(const K3E &k, const Cell &cl, const G &g, int a) {
     const int n = a == 0 ? k.nx : (a == 1 ? k.ny : k.nz);
@@ -149,25 +140,13 @@ __device__ __forceinline__ void term3(const K3E &k, const Cell &cl, int a, int s
     }
 }
 
-template <int ORDER>
-__global__ __launch_bounds__(256) void e3d_velocity_kernel(const K3E k) {
-    Cell cl;
-    if (!cell_of(k, cl)) return;
-    const long p = cl.p;
-    const float rx = k.R[0][p], ry = k.R[1][p], rz = k.R[2][p];
-    float vx = k.V[0][p], vy = k.V[1][p], vz = k.V[2][p];
-    term3(k, cl, 0, 1, RSG_E3D_SXX_LEFT, deriv<ORDER, true>(k, cl, k.Sxx, 0), vx, rx, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 1, 0, RSG_E3D_SXYY_FRONT, deriv<ORDER, false>(k, cl, k.Sxy, 1), vx, rx, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 2, 0, RSG_E3D_SXZZ_TOP, deriv<ORDER, false>(k, cl, k.Sxz, 2), vx, rx, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 0, 0, RSG_E3D_SXYX_LEFT, deriv<ORDER, false>(k, cl, k.Sxy, 0), vy, ry, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 1, 1, RSG_E3D_SYY_FRONT, deriv<ORDER, true>(k, cl, k.Syy, 1), vy, ry, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 2, 0, RSG_E3D_SYZZ_TOP, deriv<ORDER, false>(k, cl, k.Syz, 2), vy, ry, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 0, 0, RSG_E3D_SXZX_LEFT, deriv<ORDER, false>(k, cl, k.Sxz, 0), vz, rz, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 1, 0, RSG_E3D_SYZY_FRONT, deriv<ORDER, false>(k, cl, k.Syz, 1), vz, rz, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 2, 1, RSG_E3D_SZZ_TOP, deriv<ORDER, true>(k, cl, k.Szz, 2), vz, rz, nullptr, 0.f, nullptr, 0.f);
-    k.V[0][p] = vx;
-    k.V[1][p] = vy;
-    k.V[2][p] = vz;
+// forwardstepVelocity (waves.cpp:2465-2860): component a is V_a.
+template <int TX, int ORDER>
+__global__ RSG3_BOUNDS void e3d_velocity_kernel(const G3 g, const Comps3 a) {
+    using K = Div3<TX, ORDER, true, true, true, 1, false>;
+    __shared__ float lds[K::LDS];
+    Pos3 p;
+    if (tile3_of<TX>(g.t, p)) K::run(g, a.c[p.comp], p, lds);
 }
 
 // backwardstepVelocity (waves.cpp:3260-3713): the forward velocity step's
@@ -215,44 +194,6 @@ __global__ __launch_bounds__(256) void e3d_premul_kernel(const K3E k, float *w0,
     w3[p] = sxy((long)p);
     w4[p] = sxz((long)p);
     w5[p] = syz((long)p);
-}
-
-// forwardstepStress, or with BW backwardstepStress (waves.cpp:3715-4103):
-// the same terms and strips with unit moduli.
-template <int ORDER, bool BW>
-__global__ __launch_bounds__(256) void e3d_stress_kernel(const K3E k) {
-    Cell cl;
-    if (!cell_of(k, cl)) return;
-    const long p = cl.p;
-    float sxx = k.Sxx[p], syy = k.Syy[p], szz = k.Szz[p];
-    if (BW) {
-        term3(k, cl, 0, 0, RSG_E3D_VXX_LEFT, deriv<ORDER, false>(k, cl, k.V[0], 0), sxx, 1.f, nullptr, 0.f, nullptr, 0.f);
-        term3(k, cl, 1, 0, RSG_E3D_VYY_FRONT, deriv<ORDER, false>(k, cl, k.V[1], 1), syy, 1.f, nullptr, 0.f, nullptr,
-              0.f);
-        term3(k, cl, 2, 0, RSG_E3D_VZZ_TOP, deriv<ORDER, false>(k, cl, k.V[2], 2), szz, 1.f, nullptr, 0.f, nullptr, 0.f);
-    } else {
-        const float l = k.L[p], l2m = k.L2M[p];
-        term3(k, cl, 0, 0, RSG_E3D_VXX_LEFT, deriv<ORDER, false>(k, cl, k.V[0], 0), sxx, l2m, &syy, l, &szz, l);
-        term3(k, cl, 1, 0, RSG_E3D_VYY_FRONT, deriv<ORDER, false>(k, cl, k.V[1], 1), sxx, l, &syy, l2m, &szz, l);
-        term3(k, cl, 2, 0, RSG_E3D_VZZ_TOP, deriv<ORDER, false>(k, cl, k.V[2], 2), sxx, l, &syy, l, &szz, l2m);
-    }
-    // free surface: the plane lpml lies in no z strip, so zeroing after the
-    // strips is the reference's zeroing before them
-    if (k.fs && cl.c[2] == k.lpml) szz = 0.f;
-    k.Sxx[p] = sxx;
-    k.Syy[p] = syy;
-    k.Szz[p] = szz;
-    const float mxz = BW ? 1.f : k.Mxz[p], myz = BW ? 1.f : k.Myz[p], mxy = BW ? 1.f : k.Mxy[p];
-    float sxz = k.Sxz[p], syz = k.Syz[p], sxy = k.Sxy[p];
-    term3(k, cl, 0, 1, RSG_E3D_VZX_LEFT, deriv<ORDER, true>(k, cl, k.V[2], 0), sxz, mxz, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 2, 1, RSG_E3D_VXZ_TOP, deriv<ORDER, true>(k, cl, k.V[0], 2), sxz, mxz, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 2, 1, RSG_E3D_VYZ_TOP, deriv<ORDER, true>(k, cl, k.V[1], 2), syz, myz, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 1, 1, RSG_E3D_VZY_FRONT, deriv<ORDER, true>(k, cl, k.V[2], 1), syz, myz, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 1, 1, RSG_E3D_VXY_FRONT, deriv<ORDER, true>(k, cl, k.V[0], 1), sxy, mxy, nullptr, 0.f, nullptr, 0.f);
-    term3(k, cl, 0, 1, RSG_E3D_VYX_LEFT, deriv<ORDER, true>(k, cl, k.V[1], 0), sxy, mxy, nullptr, 0.f, nullptr, 0.f);
-    k.Sxz[p] = sxz;
-    k.Syz[p] = syz;
-    k.Sxy[p] = sxy;
 }
 
 // insertSource (waves.cpp:4104-4246): PRESSURE is explosive (Sxx, Syy, Szz
@@ -328,6 +269,8 @@ int check_e3d(const rsg_grid *g, const rsg_state_e3d *s) {
     if (g->nx < 2 || g->ny < 2 || g->nz < 2 || g->nz > 65535 || g->lpml < 1 || 2 * g->lpml >= g->nx ||
         2 * g->lpml >= g->ny || 2 * g->lpml >= g->nz || g->dx <= 0 || g->dy <= 0 || g->dz <= 0)
         return fail(RSG_EINVAL, "e3d: grid sizes (padded, 2 lpml < n, nz <= 65535) or steps");
+    if (g->nx >= 1 << 24 && (long long)g->nx * g->ny * 4 >= (1LL << 31))
+        return fail(RSG_EINVAL, "e3d: a tile's rows exceed 32-bit offsets (nx >= 2^24 and plane >= 2^29 cells)");
     if (!s->Vx || !s->Vy || !s->Vz || !s->Sxx || !s->Syy || !s->Szz || !s->Syz || !s->Sxz || !s->Sxy || !s->L ||
         !s->L2M || !s->Mxz || !s->Myz || !s->Mxy || !s->Rx || !s->Ry || !s->Rz || !s->tab)
         return fail(RSG_EINVAL, "e3d: null field, model or table");
@@ -384,6 +327,27 @@ K3E make_k3e(const rsg_grid *g, const rsg_state_e3d *s) {
     default: LAUNCH(8); break;  \
     }
 
+// The velocity step on six stresses (the state's own, or the weighted ones).
+int launch_velocity(const rsg_grid *g, const rsg_state_e3d *s, const float *xx, const float *yy, const float *zz,
+                    const float *yz, const float *xz, const float *xy, hipStream_t st) {
+    G3 k = make_g3e(g, s);
+    const unsigned blocks = layout3(k, 3);
+    const Comps3 a{{{{term(xx, s, RSG_E3D_SXX_LEFT, 1), term(xy, s, RSG_E3D_SXYY_FRONT, 0), term(xz, s, RSG_E3D_SXZZ_TOP, 0)},
+                     {s->Vx, nullptr, nullptr},
+                     {s->Rx, nullptr}},
+                    {{term(xy, s, RSG_E3D_SXYX_LEFT, 0), term(yy, s, RSG_E3D_SYY_FRONT, 1), term(yz, s, RSG_E3D_SYZZ_TOP, 0)},
+                     {s->Vy, nullptr, nullptr},
+                     {s->Ry, nullptr}},
+                    {{term(xz, s, RSG_E3D_SXZX_LEFT, 0), term(yz, s, RSG_E3D_SYZY_FRONT, 0), term(zz, s, RSG_E3D_SZZ_TOP, 1)},
+                     {s->Vz, nullptr, nullptr},
+                     {s->Rz, nullptr}}}};
+#define L_(X, O) e3d_velocity_kernel<X, O><<<blocks, B3, 0, st>>>(k, a)
+    RSG3_DISPATCH(k, L_)
+#undef L_
+    RSG_LAUNCH_CHECK("e3d_velocity_kernel");
+    return RSG_OK;
+}
+
 }  // namespace
 
 }  // namespace rsg
@@ -391,30 +355,17 @@ K3E make_k3e(const rsg_grid *g, const rsg_state_e3d *s) {
 namespace rsg {
 
 // backwardstepVelocity with a scratch of six padded arrays: the weighted
-// stresses once per cell, then the forward velocity kernel on them.  The
-// same values as rsg_e3d_backward_velocity, which forms them per stencil
-// point; this path reads 6 instead of up to 96 values per cell's taps.
+// stresses once per cell, then the forward velocity step on them.
 int e3d_backward_velocity_premul(const rsg_grid *g, const rsg_state_e3d *s, float *scratch, hipStream_t st) {
     if (int rc = check_e3d(g, s)) return rc;
     if (!scratch) return fail(RSG_EINVAL, "e3d: null scratch");
-    K3E k = make_k3e(g, s);
+    const K3E k = make_k3e(g, s);
     const size_t n = (size_t)g->nx * g->ny * g->nz;
     float *w[6];
     for (int i = 0; i < 6; i++) w[i] = scratch + i * n;
     e3d_premul_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(k, w[0], w[1], w[2], w[3], w[4], w[5], n);
     RSG_LAUNCH_CHECK("e3d_premul_kernel");
-    k.Sxx = w[0];
-    k.Syy = w[1];
-    k.Szz = w[2];
-    k.Sxy = w[3];
-    k.Sxz = w[4];
-    k.Syz = w[5];
-    const dim3 grid((g->nx + 63) / 64, (g->ny + 3) / 4, g->nz), block(64, 4);
-#define L_(O) e3d_velocity_kernel<O><<<grid, block, 0, st>>>(k)
-    E3D_ORDER_CASES(L_);
-#undef L_
-    RSG_LAUNCH_CHECK("e3d_velocity_kernel");
-    return RSG_OK;
+    return launch_velocity(g, s, w[0], w[1], w[2], w[5], w[4], w[3], st);
 }
 
 }  // namespace rsg
@@ -423,24 +374,12 @@ extern "C" {
 
 int rsg_e3d_forward_velocity(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
     if (int rc = rsg::check_e3d(g, s)) return rc;
-    const rsg::K3E k = rsg::make_k3e(g, s);
-    const dim3 grid((g->nx + 63) / 64, (g->ny + 3) / 4, g->nz), block(64, 4);
-#define L_(O) rsg::e3d_velocity_kernel<O><<<grid, block, 0, (hipStream_t)stream>>>(k)
-    E3D_ORDER_CASES(L_);
-#undef L_
-    RSG_LAUNCH_CHECK("e3d_velocity_kernel");
-    return RSG_OK;
+    return rsg::launch_velocity(g, s, s->Sxx, s->Syy, s->Szz, s->Syz, s->Sxz, s->Sxy, (hipStream_t)stream);
 }
 
 int rsg_e3d_forward_stress(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
     if (int rc = rsg::check_e3d(g, s)) return rc;
-    const rsg::K3E k = rsg::make_k3e(g, s);
-    const dim3 grid((g->nx + 63) / 64, (g->ny + 3) / 4, g->nz), block(64, 4);
-#define L_(O) rsg::e3d_stress_kernel<O, false><<<grid, block, 0, (hipStream_t)stream>>>(k)
-    E3D_ORDER_CASES(L_);
-#undef L_
-    RSG_LAUNCH_CHECK("e3d_stress_kernel");
-    return RSG_OK;
+    return rsg::e3d_stress_forward(g, s, (hipStream_t)stream);
 }
 
 int rsg_e3d_backward_velocity(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
@@ -460,13 +399,7 @@ int rsg_e3d_backward_velocity_ws(const rsg_grid *g, const rsg_state_e3d *s, floa
 
 int rsg_e3d_backward_stress(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
     if (int rc = rsg::check_e3d(g, s)) return rc;
-    const rsg::K3E k = rsg::make_k3e(g, s);
-    const dim3 grid((g->nx + 63) / 64, (g->ny + 3) / 4, g->nz), block(64, 4);
-#define L_(O) rsg::e3d_stress_kernel<O, true><<<grid, block, 0, (hipStream_t)stream>>>(k)
-    E3D_ORDER_CASES(L_);
-#undef L_
-    RSG_LAUNCH_CHECK("e3d_stress_kernel");
-    return RSG_OK;
+    return rsg::e3d_stress_backward(g, s, (hipStream_t)stream);
 }
 
 int rsg_e3d_insert_source(const rsg_grid *g, const rsg_state_e3d *s, const rsg_traces *src, int it, void *stream) {

@@ -8,24 +8,33 @@
 // with its halo, double buffered: one barrier a plane), the z taps from a
 // register queue of 2*ORDER values per cell.
 //
-// Everything a plane needs is loaded two planes ahead, PML memory variables
-// included, into one of two register sets.  For that to hide the latency no
-// load may be waited for early, and the compiler waits early wherever a value
-// still in flight is moved (so the queue takes its two new values at the top
-// of the next round, two planes after their loads) or wherever a branch makes
-// the number of loads in flight unknown.  So the march has no branches around
+// Everything a plane needs is loaded a plane ahead, PML memory variables
+// included, the queue's new values two.  For that to hide the latency no load
+// may be waited for early, and the compiler waits early wherever a value still
+// in flight is moved (so the queue takes its two new values at the top of the
+// next round, two planes after their loads) or wherever a branch makes the
+// number of loads in flight unknown.  So the march has no branches around
 // loads: tiles with strips or shortened stencils in x or y (PXY) and chunks
 // with them in z (PZ) are instantiations of their own, and loads past the end
-// of a chunk use an empty descriptor.
+// of a chunk use an empty descriptor.  Two planes ahead (a second set of
+// registers) costs order 8 its fourth wave a SIMD, which hides more.
 //
-// What bounds it: HBM on large grids, the march's latency (1.7 us a plane with
-// one block to a SIMD) and the filling of the queue on small ones.  Acoustic,
-// order 4, against 64 x 8 tiles that loaded one plane ahead and the memory
-// variables where they were used, us a velocity + a stress half step:
-// 320 x 300 x 280 333 + 256 -> 238 + 164 (4.5 and 3.9 TB/s algorithmic),
-// 440^3 914 + 677 -> 780 + 477, 160 x 150 x 140 66 + 58 -> 33 + 30,
-// 120 x 110 x 100 42 + 36 -> 19 + 18; order 8, 320 x 300 x 280 519 + 445 ->
-// 264 + 222.
+// What bounds it: HBM on large grids, the march's latency and the filling of
+// the queue on small ones.  Against the kernels before (acoustic: 64 x 8 tiles
+// that loaded the memory variables where they were used; elastic: a thread a
+// cell, all taps through L1 and L2), us a velocity + a stress half step:
+//   acoustic, order 4:  320 x 300 x 280  333 + 256 -> 235 + 163 (4.6, 4.0 TB/s
+//                       of its arrays once), 440^3  914 + 677 -> 769 + 467,
+//                       160 x 150 x 140  66 + 58 -> 32 + 29,
+//                       120 x 110 x 100  42 + 36 -> 19 + 18
+//   acoustic, order 8:  320 x 300 x 280  519 + 445 -> 248 + 185
+//   elastic, order 4:   200 x 190 x 180  286 + 316 -> 143 + 188,
+//                       140 x 130 x 120  80 + 85 -> 50 + 61,
+//                       70 x 60 x 50  17.2 + 17.2 -> 15.7 + 15.9
+//   elastic, order 8:   200 x 190 x 180  415 + 447 -> 177 + 218,
+//                       240^3  671 + 731 -> 287 + 371
+// The elastic steps reach 2.2 to 2.9 TB/s of their arrays once: three or four
+// blocks read each field's window and queue, from L2 for the most part.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -36,9 +45,13 @@ namespace rsg {
 
 constexpr int R3 = 2, B3 = 256;  // rows a thread, threads a block
 
-// Four waves a SIMD up to order 4 (128 VGPRs, no spills); the longer queues of
-// the higher orders need up to 168.
-#define RSG3_BOUNDS(ORDER) __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu((ORDER) <= 4 ? 4 : 3, 8)))
+// Lambdas of the march: one left out of line would put the arrays it captures,
+// the queue among them, in scratch memory.
+#define RSG_INLINE __attribute__((always_inline))
+
+// Four waves a SIMD, 128 VGPRs.  Three (168 VGPRs, two planes ahead) take 264 +
+// 222 us on 320 x 300 x 280 at order 8 where four take 248 + 185; five spill.
+#define RSG3_BOUNDS __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu(4, 8)))
 
 // Raw buffers over the tile's part of an array: every lane either has an
 // offset inside its tile's window of the grid, or kOut, which no descriptor
@@ -49,14 +62,15 @@ __device__ __forceinline__ Buf tile_buf(const float *f, long off, bool live = tr
     return mkbuf(f + off, live ? 0x7FFFFF00u : 0u);
 }
 
-// Byte offset of a plane, hidden from the optimiser: it would otherwise keep
-// one running address per array, load and store (the scalar registers then
-// spill into vector lanes) instead of two scalar adds where one is used.
+// A uniform value the optimiser may not see through (v is uniform;
+// readfirstlane says so where the compiler lost sight of it): for plane
+// offsets, where it would otherwise keep one running address per array, load
+// and store instead of two scalar adds where one is used.
 __device__ __forceinline__ long opaque(long v) {
-    asm volatile("" : "+s"(v));
-    return v;
+    int lo = __builtin_amdgcn_readfirstlane((int)v), hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return ((long)hi << 32) | (unsigned)lo;
 }
-
 // One derivative term: the field, its two strips (low, high face), and
 // whether it is the forward (1) or backward (0) difference.
 struct Term3 {
@@ -69,38 +83,46 @@ struct Term3 {
 // zones (strips or shortened stencils at the low face, neither, the high
 // face), zone i of planes z[i] .. z[i+1]-1 in n[i] chunks of zc planes; ncomp
 // components (blocks that update different arrays of one tile from partly the
-// same inputs).  With xgroups blocks are dealt round-robin to the 8 XCDs (XCD
+// same inputs), the first `first` (0 or 1) of them before all others.  With xgroups blocks are dealt round-robin to the 8 XCDs (XCD
 // k runs blocks k, k+8, ...) and XCD k marches its own contiguous group of
-// columns cg[k] .. cg[k+1]-1 through the chunks, components fastest, then
-// columns: the blocks an XCD holds at once are neighbours at the same depth,
+// columns cg[k] .. cg[k+1]-1 through the chunks, components fastest (those
+// after the first), then columns: the blocks an XCD holds at once are neighbours at the same depth,
 // so shared inputs, halos and the lines that tile rows share are fetched into
 // that XCD's L2 once.
 struct Tiles3 {
-    int tx, xgroups, ncx, ncy, zc, ncomp;
+    int tx, xgroups, ncx, ncy, zc, ncomp, first;
     int z[4], n[3];
     int cg[9];
 };
 
 struct Pos3 {
-    int x0, y0, zb, ze, comp;
-    bool pz;
+    int x0, y0, zb, ze, comp, zone;
 };
+
+// Component of block r of n blocks a component; r: its block.
+__device__ __forceinline__ bool comp_of(const Tiles3 &t, int n, int &r, int &comp) {
+    const int m = t.ncomp - t.first;
+    comp = 0;
+    if (r >= t.first * n) {
+        r -= t.first * n;
+        comp = t.first + r % m;
+        r /= m;
+    }
+    return r < n;
+}
 
 template <int TX>
 __device__ __forceinline__ bool tile3_of(const Tiles3 &t, Pos3 &p) {
     int col, ck, r = blockIdx.x;
     const int nck = t.n[0] + t.n[1] + t.n[2];
     if (!t.xgroups) {
-        p.comp = r % t.ncomp;
-        r /= t.ncomp;
+        if (!comp_of(t, t.ncx * t.ncy * nck, r, p.comp)) return false;
         ck = r / (t.ncx * t.ncy);
         col = r - ck * (t.ncx * t.ncy);
     } else {
         const int k = r % 8, ncol = t.cg[k + 1] - t.cg[k];
         r /= 8;
-        p.comp = r % t.ncomp;
-        r /= t.ncomp;
-        if (ncol <= 0 || r >= ncol * nck) return false;
+        if (ncol <= 0 || !comp_of(t, ncol * nck, r, p.comp)) return false;
         ck = r / ncol;
         col = t.cg[k] + (r - ck * ncol);
     }
@@ -118,7 +140,7 @@ __device__ __forceinline__ bool tile3_of(const Tiles3 &t, Pos3 &p) {
     }
     p.zb = t.z[zone] + ck * t.zc;
     p.ze = min(p.zb + t.zc, t.z[zone + 1]);
-    p.pz = zone != 1;
+    p.zone = zone;
     return p.zb < p.ze;
 }
 
@@ -150,6 +172,17 @@ __device__ __forceinline__ float dq(const float (&q)[2 * H + 2], const float *c)
     float acc = c[0] * (q[S + H] - q[S + H - 1]);
 #pragma unroll
     for (int io = 1; io < H; io++) acc += c[io] * (q[S + H + io] - q[S + H - 1 - io]);
+    return acc;
+}
+// The same where the array's end may shorten the stencil to order k (uniform):
+// the taps past it are masked out, whatever they hold (selects would take more
+// registers than order 8 has).
+template <int H, int S>
+__device__ __forceinline__ float dq_edge(const float (&q)[2 * H + 2], const float *c, int k) {
+    float acc = c[0] * __int_as_float(__float_as_int(q[S + H] - q[S + H - 1]) & (k > 0 ? -1 : 0));
+#pragma unroll
+    for (int io = 1; io < H; io++)
+        acc += c[io] * __int_as_float(__float_as_int(q[S + H + io] - q[S + H - 1 - io]) & (k > io ? -1 : 0));
     return acc;
 }
 template <int N>
@@ -249,23 +282,19 @@ struct Lane3 {
 #pragma unroll
         for (int r = 0; r < R3; r++) v[r] = b.ld(oc[r], 0);
     }
-    __device__ __forceinline__ void st(float *f, long o, const float (&v)[R3]) const {
-        const Buf b = tile_buf(f, o);
+    __device__ __forceinline__ void st(float *f, long o, const float (&v)[R3], bool live = true) const {
+        const Buf b = tile_buf(f, o, live);
 #pragma unroll
         for (int r = 0; r < R3; r++) b.st(v[r], oc[r], 0);
     }
-    // f at plane z of the own cells (0 outside the grid, or where not live)
-    __device__ __forceinline__ void queue(const float *f, int z, const G3 &g, float (&v)[R3], bool live = true) const {
-        const bool in = live && z >= 0 && z < g.nz;
-        ld(f, at(g, in ? z : 0), v, in);
-    }
-    // the queue before its first shift: values of planes z .. in q[2 ..] and qn
+    // the queue before its first shift: f of the own cells at planes z .. (0
+    // outside the grid) in q[2 ..] and qn
     template <int N>
     __device__ __forceinline__ void fill(const float *f, int z, const G3 &g, float (&q)[R3][N], float (&qn)[2][R3]) const {
 #pragma unroll
         for (int j = 0; j < N; j++) {
             float v[R3];
-            queue(f, z + j, g, v);
+            ld(f, at(g, z + j), v, z + j >= 0 && z + j < g.nz);
 #pragma unroll
             for (int r = 0; r < R3; r++) (j < N - 2 ? q[r][j + 2] : qn[j - (N - 2)][r]) = v[r];
         }
@@ -278,84 +307,100 @@ struct Lane3 {
 template <int TX>
 struct Sides3 {
     Face3 x, y[R3];
-    int xr;              // rows apart in an x strip (0: the second row is outside the grid)
-    long xstep, ystep;   // planes apart
-    int kx, ky[R3];      // stencil orders
+    bool inx[R3];
+    bool px, py, ex, ey;  // does the tile (uniform) hold cells of x / y strips, of shortened x / y stencils?
+    int xr;               // rows apart in an x strip (0: the second row is outside the grid)
+    long xstep, ystep;    // planes apart
+    int kx, ky[R3];       // stencil orders
     __device__ __forceinline__ void init(const G3 &g, const Pos3 &p, const Lane3<TX> &ln, const Term3 &tx, const Term3 &ty) {
+        constexpr int TY = R3 * B3 / TX;
         const int nx = g.nx, ny = g.ny, L = g.lpml, H = g.order;
+        px = p.x0 < L || p.x0 + TX > nx - L;
+        py = p.y0 < L || p.y0 + TY > ny - L;
+        ex = p.x0 < H || p.x0 + TX > nx - H;
+        ey = p.y0 < H || p.y0 + TY > ny - H;
         xstep = (long)ny * L;
         ystep = (long)L * nx;
         const int xc = min(ln.x, nx - 1), yc = min(ln.y, ny - 1);
         xr = ln.ok[1] ? L : 0;
         if (tx.f)
-            x.init(xc, nx, L, ln.ok[0], tx.lo, tx.hi, [&](int j) { return p.zb * xstep + (long)yc * L + j; }, g.tab, tx.fw);
+            x.init(xc, nx, L, ln.ok[0], tx.lo, tx.hi, [&](int j) RSG_INLINE { return p.zb * xstep + (long)yc * L + j; }, g.tab, tx.fw);
         kx = tx.fw ? kfw(ln.x, nx, H) : kbw(ln.x, nx, H);
 #pragma unroll
         for (int r = 0; r < R3; r++) {
+            inx[r] = tx.f && x.in && ln.ok[r];
             if (ty.f)
                 y[r].init(min(ln.y + r, ny - 1), ny, L, ln.ok[r], ty.lo, ty.hi,
-                          [&](int j) { return p.zb * ystep + (long)j * nx + xc; }, g.tab, ty.fw);
+                          [&](int j) RSG_INLINE { return p.zb * ystep + (long)j * nx + xc; }, g.tab, ty.fw);
             ky[r] = ty.fw ? kfw(ln.y + r, ny, H) : kbw(ln.y + r, ny, H);
         }
+        xstep = opaque(xstep);
+        ystep = opaque(ystep);
     }
-    // memory variables k planes on
-    __device__ __forceinline__ void load_x(float (&v)[R3], int k) const {
+    // memory variables `at` values on from the strips' current plane
+    __device__ __forceinline__ void load_x(float (&v)[R3], long at) const {
 #pragma unroll
-        for (int r = 0; r < R3; r++) v[r] = x.psi[k * xstep + r * xr];
+        for (int r = 0; r < R3; r++) v[r] = x.psi[at + r * xr];
     }
-    __device__ __forceinline__ void load_y(float (&v)[R3], int k) const {
+    __device__ __forceinline__ void load_y(float (&v)[R3], long at) const {
 #pragma unroll
-        for (int r = 0; r < R3; r++) v[r] = y[r].psi[k * ystep];
+        for (int r = 0; r < R3; r++) v[r] = y[r].psi[at];
     }
-    __device__ __forceinline__ bool in_x(const Lane3<TX> &ln, int r) const { return x.in && ln.ok[r]; }
-    __device__ __forceinline__ void next() {
-        x.psi += 2 * xstep;
+    __device__ __forceinline__ void store_x(const float (&v)[R3], long at) const {
 #pragma unroll
-        for (int r = 0; r < R3; r++) y[r].psi += 2 * ystep;
+        for (int r = 0; r < R3; r++)
+            if (inx[r]) x.psi[at + r * xr] = v[r];
+    }
+    __device__ __forceinline__ void store_y(const float (&v)[R3], long at) const {
+#pragma unroll
+        for (int r = 0; r < R3; r++)
+            if (y[r].in) y[r].psi[at] = v[r];
     }
 };
 
-// The z strips of a plane: memory variables of the own cells and the plane's
-// profile values.  A plane between the strips (a PZ chunk of a grid whose
-// strips are thinner than the stencil) loads nothing and has in = false.
-struct ZPml {
-    float A, B, C, v[R3];
-    __device__ __forceinline__ static bool inside(const G3 &g, int z, bool &h, int &j) {
-        h = z >= g.nz - g.lpml;
-        j = h ? z - (g.nz - g.lpml) : z;
-        return z < g.lpml || h;
+// The z strip of a PZ chunk (one face): the memory variables of its planes'
+// own cells and their profile values.  A plane between the strips (of a grid
+// whose strips are thinner than the stencil) loads and stores nothing.
+struct ZStrip {
+    float *psi;
+    const float *tab;
+    int L, z0;  // strip plane of z: z - z0
+    __device__ __forceinline__ void init(const G3 &g, const Pos3 &p, const Term3 &t) {
+        const bool h = p.zone == 2;
+        L = g.lpml;
+        z0 = h ? g.nz - L : 0;
+        psi = h ? t.hi : t.lo;
+        tab = g.tab + ((h ? T_RBB : 0) + t.fw * T_STAG) * L;
     }
-    template <int TX>
-    __device__ __forceinline__ void load(const G3 &g, const Term3 &t, int z, const Lane3<TX> &ln, bool live) {
-        bool h;
-        int j;
-        const bool in = inside(g, z, h, j) && live;
-        const float *tb = g.tab + ((h ? T_RBB : 0) + t.fw * T_STAG) * g.lpml + (in ? j : 0);
-        A = tb[T_A * g.lpml];
-        B = tb[T_B * g.lpml];
-        C = tb[T_C * g.lpml];
-        ln.ld(h ? t.hi : t.lo, opaque((in ? j : 0) * ((long)g.nx * g.ny) + ln.t0), v, in);
-    }
-    template <int TX>
-    __device__ __forceinline__ void store(const G3 &g, const Term3 &t, int z, const Lane3<TX> &ln) const {
-        bool h;
-        int j;
-        const bool in = inside(g, z, h, j);
-        const Buf b = tile_buf(h ? t.hi : t.lo, opaque((in ? j : 0) * ((long)g.nx * g.ny) + ln.t0), in);
-#pragma unroll
-        for (int r = 0; r < R3; r++) b.st(v[r], ln.oc[r], 0);
-    }
+    __device__ __forceinline__ bool in(int z) const { return z >= z0 && z < z0 + L; }
 };
+struct ZVals {
+    float A, B, C, v[R3];
+};
+template <int TX>
+__device__ __forceinline__ void zload(ZVals &v, const ZStrip &s, const G3 &g, int z, const Lane3<TX> &ln, bool live) {
+    const bool in = s.in(z) && live;
+    const int j = in ? z - s.z0 : 0;
+    v.A = s.tab[T_A * s.L + j];
+    v.B = s.tab[T_B * s.L + j];
+    v.C = s.tab[T_C * s.L + j];
+    ln.ld(s.psi, j * ((long)g.nx * g.ny) + ln.t0, v.v, in);
+}
+template <int TX>
+__device__ __forceinline__ void zstore(const ZVals &v, const ZStrip &s, const G3 &g, int z, const Lane3<TX> &ln) {
+    const bool in = s.in(z);
+    ln.st(s.psi, (in ? z - s.z0 : 0) * ((long)g.nx * g.ny) + ln.t0, v.v, in);
+}
 
 // psi = B psi + A d; F -= m (psi + C d) for a cell in the strip.
 __device__ __forceinline__ void strip3(float &F, float m, float d, bool in, float C, float psi) {
     F = in ? F - m * (psi + C * d) : F;
 }
 
-// Two planes a round: body(S, z) for the even (S = 0) and odd (S = 1) planes
-// of [zb, ze), top(z) before each pair, next() after it.
-template <class T, class B, class N>
-__device__ __forceinline__ void march3(int zb, int ze, T &&top, B &&body, N &&next) {
+// Two planes a round: top(z) before each pair, then body(S, z) for the even
+// (S = 0) and the odd (S = 1) plane of the chunk.
+template <class T, class B>
+__device__ __forceinline__ void march3(int zb, int ze, T &&top, B &&body) {
     constexpr std::integral_constant<int, 0> S0;
     constexpr std::integral_constant<int, 1> S1;
 #pragma unroll 1
@@ -364,7 +409,6 @@ __device__ __forceinline__ void march3(int zb, int ze, T &&top, B &&body, N &&ne
         body(S0, z);
         if (z + 1 >= ze) break;
         body(S1, z + 1);
-        next();
         z += 2;
         if (z >= ze) break;
     }
@@ -384,7 +428,7 @@ struct Comp3 {
     const float *M[2];  // the modulus (NOUT 1), or L, L + 2 mu
 };
 
-template <int TX, int ORDER, bool HX, bool HY, bool HZ, int NOUT, bool UNIT>
+template <int TX, int ORDER, bool HX, bool HY, bool HZ, int NOUT, bool UNIT, bool FULL = true>
 struct Div3 {
     static constexpr int H = ORDER, NM = UNIT ? 0 : (NOUT == 3 ? 2 : 1);
     using WX = Win3<TX, H, 0>;
@@ -394,7 +438,7 @@ struct Div3 {
 
     template <bool PXY, bool PZ>
     static __device__ __forceinline__ void march(const G3 &g, const Comp3 &c, const Pos3 &p, float *lds) {
-        const int fx = c.t[0].fw, fy = c.t[1].fw, fz = c.t[2].fw, nx = g.nx;
+        const int fx = c.t[0].fw, fy = c.t[1].fw, fz = c.t[2].fw, nx = g.nx, ze = p.ze;
         const Lane3<TX> ln(g, p);
         float *const ce = lds + 2 * (LX + LY);
         WX wx;
@@ -402,138 +446,139 @@ struct Div3 {
         if (HX) wx.init(nx, g.ny, p.x0, p.y0);
         if (HY) wy.init(nx, g.ny, p.x0, p.y0);
         Sides3<TX> sd;
+        ZStrip zs;
         if (PXY) {
             sd.init(g, p, ln, c.t[0], c.t[1]);
             if (threadIdx.x < 36) ce[threadIdx.x] = kCoefC[threadIdx.x];
         }
-        // two sets of a plane's values (even and odd planes of the chunk)
-        float F[2][NOUT][R3], M[2][NM ? NM : 1][R3], sx[2][R3], sy[2][R3], q[R3][2 * H + 2], qn[2][R3];
-        float wvx[2][WX::K], wvy[2][WY::K];
-        ZPml zp[2];
-        auto window = [&](auto S, int z) {
-            constexpr int s = decltype(S)::value;
-            const bool live = z < p.ze;
-            const long at = ln.at(g, live ? z : 0);
-            if (HX) wx.fetch(wvx[s], c.t[0].f, at, nx, live);
-            if (HY) wy.fetch(wvy[s], c.t[1].f, at, nx, live);
-        };
-        // the own cells and memory variables of plane z, k planes from the
-        // strips' current one
-        auto own = [&](auto S, int z, int k) {
-            constexpr int s = decltype(S)::value;
-            const bool live = z < p.ze;
-            const long at = ln.at(g, live ? z : 0);
+        if (PZ && HZ) zs.init(g, p, c.t[2]);
+        const float *const f[3] = {c.t[0].f, c.t[1].f, c.t[2].f};
+        float *Fp[NOUT];
+        const float *Mp[NM ? NM : 1];
 #pragma unroll
-            for (int i = 0; i < NOUT; i++) ln.ld(c.F[i], at, F[s][i], live);
+        for (int i = 0; i < NOUT; i++) Fp[i] = c.F[i];
 #pragma unroll
-            for (int i = 0; i < NM; i++) ln.ld(c.M[i], at, M[s][i], live);
-            if (PXY && HX) sd.load_x(sx[s], live ? k : 0);
-            if (PXY && HY) sd.load_y(sy[s], live ? k : 0);
-            if (PZ && HZ) zp[s].load(g, c.t[2], z, ln, live);
+        for (int i = 0; i < NM; i++) Mp[i] = c.M[i];
+        const long nxy = opaque((long)nx * g.ny);
+        long o = ln.at(g, p.zb);      // the current plane's part of the tile
+        long xo = 0, yo = 0;          // and of its strips
+        // the next plane's values, once the current plane's are used
+        float F[NOUT][R3], M[NM ? NM : 1][R3], sx[R3], sy[R3], q[R3][2 * H + 2], qn[2][R3], wvx[WX::K], wvy[WY::K];
+        ZVals zv;
+        // plane z, k planes after the current one
+        auto window = [&](int z, int k) RSG_INLINE {
+            const bool live = z < ze;
+            const long at = opaque(o + k * nxy);
+            if (HX) wx.fetch(wvx, f[0], at, nx, live);
+            if (HY) wy.fetch(wvy, f[1], at, nx, live);
         };
-        constexpr std::integral_constant<int, 0> S0;
-        constexpr std::integral_constant<int, 1> S1;
-        if (HZ) ln.fill(c.t[2].f, p.zb + fz - H, g, q, qn);
-        window(S0, p.zb);
-        own(S0, p.zb, 0);
-        window(S1, p.zb + 1);
-        own(S1, p.zb + 1, 1);
-        auto top = [&](int z) {
+        auto own = [&](int z, int k) RSG_INLINE {
+            const bool live = z < ze;
+            const long at = opaque(o + k * nxy);
+#pragma unroll
+            for (int i = 0; i < NOUT; i++) ln.ld(Fp[i], at, F[i], live);
+#pragma unroll
+            for (int i = 0; i < NM; i++) ln.ld(Mp[i], at, M[i], live);
+            if (PXY && HX) sd.load_x(sx, xo + (live ? k * sd.xstep : 0));
+            if (PXY && HY) sd.load_y(sy, yo + (live ? k * sd.ystep : 0));
+            if (PZ && HZ) zload(zv, zs, g, z, ln, live);
+        };
+        if (HZ) ln.fill(f[2], p.zb + fz - H, g, q, qn);
+        window(p.zb, 0);
+        own(p.zb, 0);
+        const int qz = fz + H;  // the queue's next plane, from two planes on
+        auto top = [&](int z) RSG_INLINE {
+            o = opaque(o);
             if (HZ) {
                 shift2(q, qn);
-                ln.queue(c.t[2].f, z + 2 + fz + H, g, qn[0], z + 2 < p.ze);
-                ln.queue(c.t[2].f, z + 3 + fz + H, g, qn[1], z + 3 < p.ze);
+                ln.ld(f[2], o + (qz + 2) * nxy, qn[0], z + 2 < ze && z + 2 + qz < g.nz);
+                ln.ld(f[2], o + (qz + 3) * nxy, qn[1], z + 3 < ze && z + 3 + qz < g.nz);
             }
         };
-        auto body = [&](auto S, int z) {
-            constexpr int s = decltype(S)::value;
-            float *const bx = lds + s * (LX + LY), *const by = bx + LX;
-            if (HX) wx.store(wvx[s], bx);
-            if (HY) wy.store(wvy[s], by);
+        auto body = [&](auto S, int z) RSG_INLINE {
+            constexpr int sb = decltype(S)::value;
+            float *const bx = lds + sb * (LX + LY), *const by = bx + LX;
+            if (HX) wx.store(wvx, bx);
+            if (HY) wy.store(wvy, by);
             __syncthreads();
-            window(S, z + 2);
-            float cz[H];
-#pragma unroll
-            for (int i = 0; i < H; i++) cz[i] = PZ ? g.cz[fz ? kfw(z, g.nz, H) : kbw(z, g.nz, H)][i] : g.c[2][i];
-            bool zh;
-            int zj;
-            const bool zin = PZ && ZPml::inside(g, z, zh, zj);
+            window(z + 1, 1);
+            const int kz = PZ ? (fz ? kfw(z, g.nz, H) : kbw(z, g.nz, H)) : H;
+            const float *const cz = g.cz[kz];
+            const bool zin = PZ && HZ && zs.in(z);
 #pragma unroll
             for (int r = 0; r < R3; r++) {
                 const int yl = ln.ty * R3 + r;
-                auto m = [&](int a, int i) { return UNIT ? g.dt : g.dt * M[s][NOUT == 3 && i == a ? NM - 1 : 0][r]; };
-                auto plain = [&](int a, float d) {
+                auto m = [&](int a, int i) RSG_INLINE { return UNIT ? g.dt : g.dt * M[NOUT == 3 && i == a ? NM - 1 : 0][r]; };
+                auto plain = [&](int a, float d) RSG_INLINE {
 #pragma unroll
                     for (int i = 0; i < NOUT; i++)
-                        if (!(NOUT == 3 && UNIT && i != a)) F[s][i][r] += m(a, i) * d;
+                        if (!(NOUT == 3 && UNIT && i != a)) F[i][r] += m(a, i) * d;
                 };
-                auto strip = [&](int a, float d, bool in, float C, float psi) {
+                auto strip = [&](int a, float d, bool in, float C, float psi) RSG_INLINE {
 #pragma unroll
                     for (int i = 0; i < NOUT; i++)
-                        if (!(NOUT == 3 && UNIT && i != a)) strip3(F[s][i][r], m(a, i), d, in, C, psi);
+                        if (!(NOUT == 3 && UNIT && i != a)) strip3(F[i][r], m(a, i), d, in, C, psi);
                 };
                 if (HX) {
                     // the backward difference is the forward one a cell before
                     const float *w = bx + yl * WX::LD + ln.tx + H - 1 + fx;
                     float d = dfw<ORDER>(w, 1, g.c[0]);
-                    if (PXY && sd.kx != H) d = dfw_edge(w, 1, sd.kx, g.inv[0], ce);
+                    if (PXY && sd.ex)
+                        if (sd.kx != H) d = dfw_edge(w, 1, sd.kx, g.inv[0], ce);
                     plain(0, d);
-                    if (PXY) {
-                        sx[s][r] = sd.x.B * sx[s][r] + sd.x.A * d;
-                        strip(0, d, sd.in_x(ln, r), sd.x.C, sx[s][r]);
+                    if (PXY && sd.px) {
+                        sx[r] = sd.x.B * sx[r] + sd.x.A * d;
+                        strip(0, d, sd.inx[r], sd.x.C, sx[r]);
                     }
                 }
                 if (HY) {
                     const float *w = by + (yl + H - 1 + fy) * WY::LD + ln.tx;
                     float d = dfw<ORDER>(w, WY::LD, g.c[1]);
-                    if (PXY && sd.ky[r] != H) d = dfw_edge(w, WY::LD, sd.ky[r], g.inv[1], ce);
+                    if (PXY && sd.ey)
+                        if (sd.ky[r] != H) d = dfw_edge(w, WY::LD, sd.ky[r], g.inv[1], ce);
                     plain(1, d);
-                    if (PXY) {
-                        sy[s][r] = sd.y[r].B * sy[s][r] + sd.y[r].A * d;
-                        strip(1, d, sd.y[r].in, sd.y[r].C, sy[s][r]);
+                    if (PXY && sd.py) {
+                        sy[r] = sd.y[r].B * sy[r] + sd.y[r].A * d;
+                        strip(1, d, sd.y[r].in, sd.y[r].C, sy[r]);
                     }
                 }
                 if (HZ) {
-                    const float d = dq<H, s>(q[r], cz);
+                    const float d = PZ ? dq_edge<H, sb>(q[r], cz, kz) : dq<H, sb>(q[r], g.c[2]);
                     plain(2, d);
-                    if (PZ) {
-                        zp[s].v[r] = zp[s].B * zp[s].v[r] + zp[s].A * d;
-                        strip(2, d, zin, zp[s].C, zp[s].v[r]);
+                    if (PZ && zin) {
+                        zv.v[r] = zv.B * zv.v[r] + zv.A * d;
+                        strip(2, d, true, zv.C, zv.v[r]);
                     }
                 }
                 // free surface: the plane lpml lies in no z strip, so zeroing
                 // after the strips is the reference's zeroing before them
-                if (NOUT == 3 && g.fs && z == g.lpml) F[s][NOUT - 1][r] = 0.f;
+                if (NOUT == 3 && g.fs && z == g.lpml) F[NOUT - 1][r] = 0.f;
             }
-            const long at = ln.at(g, z);
 #pragma unroll
-            for (int i = 0; i < NOUT; i++) ln.st(c.F[i], at, F[s][i]);
-            if (PZ && HZ) zp[s].store(g, c.t[2], z, ln);
-            if (PXY)
-#pragma unroll
-                for (int r = 0; r < R3; r++) {
-                    if (HX && sd.in_x(ln, r)) sd.x.psi[s * sd.xstep + r * sd.xr] = sx[s][r];
-                    if (HY && sd.y[r].in) sd.y[r].psi[s * sd.ystep] = sy[s][r];
-                }
-            own(S, z + 2, s + 2);
+            for (int i = 0; i < NOUT; i++) ln.st(Fp[i], o, F[i]);
+            if (PZ && HZ) zstore(zv, zs, g, z, ln);
+            if (PXY && HX && sd.px) sd.store_x(sx, xo);
+            if (PXY && HY && sd.py) sd.store_y(sy, yo);
+            own(z + 1, 1);
+            o += nxy;
+            if (PXY) {
+                xo += sd.xstep;
+                yo += sd.ystep;
+            }
         };
-        march3(p.zb, p.ze, top, body, [&]() {
-            if (PXY) sd.next();
-        });
+        march3(p.zb, ze, top, body);
     }
 
     static __device__ __forceinline__ void run(const G3 &g, const Comp3 &c, const Pos3 &p, float *lds) {
-        if (tile_pxy<TX>(g, p)) {
-            if (p.pz && HZ)
-                march<true, true>(g, c, p, lds);
-            else
-                march<true, false>(g, c, p, lds);
-        } else {
-            if (p.pz && HZ)
-                march<false, true>(g, c, p, lds);
-            else
-                march<false, false>(g, c, p, lds);
-        }
+        const bool pxy = tile_pxy<TX>(g, p), pz = p.zone != 1;
+        if (FULL && pxy && !pz)
+            march<true, false>(g, c, p, lds);
+        else if (FULL && HZ && pz && !pxy)
+            march<false, true>(g, c, p, lds);
+        else if (pxy || pz)
+            march<true, true>(g, c, p, lds);
+        else
+            march<false, false>(g, c, p, lds);
     }
 };
 
@@ -556,113 +601,111 @@ struct Grad3 {
 
     template <bool PXY, bool PZ>
     static __device__ __forceinline__ void march(const G3 &g, const Grad3Args &c, const Pos3 &p, float *lds) {
-        const float *P = c.t[0].f;
+        const int nx = g.nx, ze = p.ze;
         const Lane3<TX> ln(g, p);
-        const int nx = g.nx;
         float *const ce = lds + 2 * W::N;
         W w;
         w.init(nx, g.ny, p.x0, p.y0);
         Sides3<TX> sd;
+        ZStrip zs;
         if (PXY) {
             sd.init(g, p, ln, c.t[0], c.t[1]);
             if (threadIdx.x < 36) ce[threadIdx.x] = kCoefC[threadIdx.x];
         }
-        float V[2][3][R3], R[2][3][R3], sx[2][R3], sy[2][R3], wv[2][W::K], q[R3][2 * H + 2], qn[2][R3];
-        ZPml zp[2];
-        auto window = [&](auto S, int z) {
-            const bool live = z < p.ze;
-            w.fetch(wv[decltype(S)::value], P, ln.at(g, live ? z : 0), nx, live);
+        if (PZ) zs.init(g, p, c.t[2]);
+        const float *const P = c.t[0].f;
+        float *const Vp[3] = {c.V[0], c.V[1], c.V[2]};
+        const float *const Rp[3] = {c.R[0], c.R[1], c.R[2]};
+        const long nxy = opaque((long)nx * g.ny);
+        long o = ln.at(g, p.zb), xo = 0, yo = 0;
+        float V[3][R3], R[3][R3], sx[R3], sy[R3], wv[W::K], q[R3][2 * H + 2], qn[2][R3];
+        ZVals zv;
+        auto window = [&](int z, int k) RSG_INLINE {
+            w.fetch(wv, P, opaque(o + k * nxy), nx, z < ze);
         };
-        auto own = [&](auto S, int z, int k) {
-            constexpr int s = decltype(S)::value;
-            const bool live = z < p.ze;
-            const long at = ln.at(g, live ? z : 0);
+        auto own = [&](int z, int k) RSG_INLINE {
+            const bool live = z < ze;
+            const long at = opaque(o + k * nxy);
 #pragma unroll
             for (int a = 0; a < 3; a++) {
-                ln.ld(c.V[a], at, V[s][a], live);
-                ln.ld(c.R[a], at, R[s][a], live);
+                ln.ld(Vp[a], at, V[a], live);
+                ln.ld(Rp[a], at, R[a], live);
             }
             if (PXY) {
-                sd.load_x(sx[s], live ? k : 0);
-                sd.load_y(sy[s], live ? k : 0);
+                sd.load_x(sx, xo + (live ? k * sd.xstep : 0));
+                sd.load_y(sy, yo + (live ? k * sd.ystep : 0));
             }
-            if (PZ) zp[s].load(g, c.t[2], z, ln, live);
+            if (PZ) zload(zv, zs, g, z, ln, live);
         };
-        constexpr std::integral_constant<int, 0> S0;
-        constexpr std::integral_constant<int, 1> S1;
         ln.fill(P, p.zb + 1 - H, g, q, qn);
-        window(S0, p.zb);
-        own(S0, p.zb, 0);
-        window(S1, p.zb + 1);
-        own(S1, p.zb + 1, 1);
-        auto top = [&](int z) {
+        window(p.zb, 0);
+        own(p.zb, 0);
+        auto top = [&](int z) RSG_INLINE {
+            o = opaque(o);
             shift2(q, qn);
-            ln.queue(P, z + 3 + H, g, qn[0], z + 2 < p.ze);
-            ln.queue(P, z + 4 + H, g, qn[1], z + 3 < p.ze);
+            ln.ld(P, o + (H + 3) * nxy, qn[0], z + 2 < ze && z + 3 + H < g.nz);
+            ln.ld(P, o + (H + 4) * nxy, qn[1], z + 3 < ze && z + 4 + H < g.nz);
         };
-        auto body = [&](auto S, int z) {
-            constexpr int s = decltype(S)::value;
-            float *const b = lds + s * W::N;
-            w.store(wv[s], b);
+        auto body = [&](auto S, int z) RSG_INLINE {
+            constexpr int sb = decltype(S)::value;
+            float *const b = lds + sb * W::N;
+            w.store(wv, b);
             __syncthreads();
-            window(S, z + 2);
-            float cz[H];
-#pragma unroll
-            for (int i = 0; i < H; i++) cz[i] = PZ ? g.cz[kfw(z, g.nz, H)][i] : g.c[2][i];
-            bool zh;
-            int zj;
-            const bool zin = PZ && ZPml::inside(g, z, zh, zj);
+            window(z + 1, 1);
+            const int kz = PZ ? kfw(z, g.nz, H) : H;
+            const float *const cz = g.cz[kz];
+            const bool zin = PZ && zs.in(z);
 #pragma unroll
             for (int r = 0; r < R3; r++) {
                 const float *t = b + (ln.ty * R3 + r + H) * W::LD + ln.tx + H;
-                float m = g.dt * R[s][0][r], d = dfw<ORDER>(t, 1, g.c[0]);
-                if (PXY && sd.kx != H) d = dfw_edge(t, 1, sd.kx, g.inv[0], ce);
-                V[s][0][r] += m * d;
-                if (PXY) {
-                    sx[s][r] = sd.x.B * sx[s][r] + sd.x.A * d;
-                    strip3(V[s][0][r], m, d, sd.in_x(ln, r), sd.x.C, sx[s][r]);
+                float m = g.dt * R[0][r], d = dfw<ORDER>(t, 1, g.c[0]);
+                if (PXY && sd.ex)
+                    if (sd.kx != H) d = dfw_edge(t, 1, sd.kx, g.inv[0], ce);
+                V[0][r] += m * d;
+                if (PXY && sd.px) {
+                    sx[r] = sd.x.B * sx[r] + sd.x.A * d;
+                    strip3(V[0][r], m, d, sd.inx[r], sd.x.C, sx[r]);
                 }
-                m = g.dt * R[s][1][r];
+                m = g.dt * R[1][r];
                 d = dfw<ORDER>(t, W::LD, g.c[1]);
-                if (PXY && sd.ky[r] != H) d = dfw_edge(t, W::LD, sd.ky[r], g.inv[1], ce);
-                V[s][1][r] += m * d;
-                if (PXY) {
-                    sy[s][r] = sd.y[r].B * sy[s][r] + sd.y[r].A * d;
-                    strip3(V[s][1][r], m, d, sd.y[r].in, sd.y[r].C, sy[s][r]);
+                if (PXY && sd.ey)
+                    if (sd.ky[r] != H) d = dfw_edge(t, W::LD, sd.ky[r], g.inv[1], ce);
+                V[1][r] += m * d;
+                if (PXY && sd.py) {
+                    sy[r] = sd.y[r].B * sy[r] + sd.y[r].A * d;
+                    strip3(V[1][r], m, d, sd.y[r].in, sd.y[r].C, sy[r]);
                 }
-                m = g.dt * R[s][2][r];
-                d = dq<H, s>(q[r], cz);
-                V[s][2][r] += m * d;
-                if (PZ) {
-                    zp[s].v[r] = zp[s].B * zp[s].v[r] + zp[s].A * d;
-                    strip3(V[s][2][r], m, d, zin, zp[s].C, zp[s].v[r]);
+                m = g.dt * R[2][r];
+                d = PZ ? dq_edge<H, sb>(q[r], cz, kz) : dq<H, sb>(q[r], g.c[2]);
+                V[2][r] += m * d;
+                if (PZ && zin) {
+                    zv.v[r] = zv.B * zv.v[r] + zv.A * d;
+                    strip3(V[2][r], m, d, true, zv.C, zv.v[r]);
                 }
             }
-            const long at = ln.at(g, z);
 #pragma unroll
-            for (int a = 0; a < 3; a++) ln.st(c.V[a], at, V[s][a]);
-            if (PZ) zp[s].store(g, c.t[2], z, ln);
-            if (PXY)
-#pragma unroll
-                for (int r = 0; r < R3; r++) {
-                    if (sd.in_x(ln, r)) sd.x.psi[s * sd.xstep + r * sd.xr] = sx[s][r];
-                    if (sd.y[r].in) sd.y[r].psi[s * sd.ystep] = sy[s][r];
-                }
-            own(S, z + 2, s + 2);
+            for (int a = 0; a < 3; a++) ln.st(Vp[a], o, V[a]);
+            if (PZ) zstore(zv, zs, g, z, ln);
+            if (PXY && sd.px) sd.store_x(sx, xo);
+            if (PXY && sd.py) sd.store_y(sy, yo);
+            own(z + 1, 1);
+            o += nxy;
+            if (PXY) {
+                xo += sd.xstep;
+                yo += sd.ystep;
+            }
         };
-        march3(p.zb, p.ze, top, body, [&]() {
-            if (PXY) sd.next();
-        });
+        march3(p.zb, ze, top, body);
     }
 
     static __device__ __forceinline__ void run(const G3 &g, const Grad3Args &c, const Pos3 &p, float *lds) {
         if (tile_pxy<TX>(g, p)) {
-            if (p.pz)
+            if (p.zone != 1)
                 march<true, true>(g, c, p, lds);
             else
                 march<true, false>(g, c, p, lds);
         } else {
-            if (p.pz)
+            if (p.zone != 1)
                 march<false, true>(g, c, p, lds);
             else
                 march<false, false>(g, c, p, lds);
@@ -697,7 +740,7 @@ static G3 make_g3(const rsg_grid *g, const float *tab, int order) {
 }
 
 // Launch grid of ncomp components, and the tile order.
-static unsigned layout3(G3 &k, int ncomp) {
+static unsigned layout3(G3 &k, int ncomp, int first = 0) {
     Tiles3 &t = k.t;
     // Rows of 64 touch fewer partly used cache lines (440^3, order 4: 778 + 474
     // us a step against 873 + 514 with 32), unless they waste much more of a
@@ -708,7 +751,9 @@ static unsigned layout3(G3 &k, int ncomp) {
     t.ncx = (k.nx + t.tx - 1) / t.tx;
     t.ncy = (k.ny + ty - 1) / ty;
     t.ncomp = ncomp;
-    const int m = std::max(k.lpml, k.order), lo = std::min(m, k.nz), hi = std::max(lo, k.nz - m);
+    t.first = first;
+    // the low zone ends before the high strip, so that a chunk has one face
+    const int m = std::max(k.lpml, k.order), lo = std::min(m, k.nz - k.lpml), hi = std::max(lo, k.nz - m);
     t.z[0] = 0;
     t.z[1] = lo;
     t.z[2] = hi;
@@ -722,10 +767,13 @@ static unsigned layout3(G3 &k, int ncomp) {
     int zc = tuning().zc3d;
     if (zc <= 0) {
         // Short chunks give many blocks, long ones amortise the queue's
-        // filling: 8 planes where that gives four rounds of blocks (320 x 300 x
-        // 280: 230 + 155 us a step with 8, 235 + 158 with 12, 250 + 169 with
-        // 24), else 4 (120 x 110 x 100: 19 + 18 us with 4, 21 + 22 with 8).
-        zc = cols * split(8) >= 4096 ? 8 : 4;
+        // filling: 8 planes where that gives enough blocks, else 4.  One
+        // component: four rounds (320 x 300 x 280: 229 + 154 us a step with 8,
+        // 230 + 161 with 4; 200 x 190 x 180, 2400 blocks: 69 + 50 with 8, 62 +
+        // 50 with 4).  The elastic components' blocks do less each and start
+        // cheaper on lines their neighbours read: two rounds (140 x 130 x 120:
+        // 50 + 60 us with 8, 53 + 64 with 4; 70 x 60 x 50: 21 + 23, 16 + 16).
+        zc = cols * split(8) >= (ncomp > 1 ? 2048 : 4096) ? 8 : 4;
     }
     const int nck = split(zc), ncol = t.ncx * t.ncy;
     t.xgroups = tuning().xcd3d ? 1 : 0;
