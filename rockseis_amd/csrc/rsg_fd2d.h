@@ -48,11 +48,15 @@ __device__ __forceinline__ void cell_st(const Buf &b, float v, unsigned cb, int 
 constexpr int BX = 64;
 constexpr int BZ = 4;
 
+// Row of the block a thread works in: one per wavefront, so everything derived
+// from it alone (rows' strips, orders, offsets) is uniform and stays scalar.
+__device__ __forceinline__ int block_row() { return __builtin_amdgcn_readfirstlane((int)threadIdx.y); }
+
 // Source injection and velocity gathers done by the stress kernel itself
 // (insertSource / recordData of the same time step, waves.cpp:407-595,
 // 2085-2288), so a modelling step is two launches: each stress-type source
-// cell is updated by the thread that owns it, right after its stress update,
-// traces in order (the reference's serial order); each velocity receiver is
+// cell is updated by the thread that owns it, in its registers right after its
+// stress update, traces in order (the reference's serial order); each velocity receiver is
 // gathered by one thread of the block whose tile holds its base cell, from
 // that block's LDS tiles of Vx and Vz (the velocities of the step are final
 // and the tiles carry a halo on both axes).
@@ -97,27 +101,42 @@ struct K2D {
     FusedIO io;  // stress kernels of single-shot modelling runs only
 };
 
-// Injection of the fused sources, run by each thread after it has stored
-// its updated stress cells (column x, rows zt .. zt+RZ-1 at byte offset cb,
-// rows rowb apart): F += ((scale * modulus) * w) * xtri * ytri at every
-// source corner among them, traces in order (the cell was written by this
-// same thread, so reading it back is ordered).  Mod null: modulus 1; F2 set:
-// the same term into F2 (elastic explosive source, Sxx and Szz).
-template <int RZ, bool FAST>
-__device__ __forceinline__ void fused_inject(const FusedIO &io, const Buf &bF, const Buf *bF2, const Buf *bMod,
-                                          int x, int zt, int nz, unsigned cb, int rowb, int it) {
-    for (int i = 0; i < io.nsrc; i++) {
-        const int i2 = x - io.sx[i];
-        if (io.sx[i] < 0 || i2 < 0 || i2 > 1) continue;
-        const float w = io.wav[(size_t)i * io.src_nt + it];
-        for (int i1 = 0; i1 < 2; i1++) {
-            const int r = io.sz[i] + i1 - zt;
-            if (r < 0 || r >= RZ || zt + r >= nz) continue;
-            const float m = bMod ? io.scale * cell_ld<FAST>(*bMod, cb, r, rowb) : io.scale;
-            const float v = m * w * io.wx[i][i2] * io.wz[i][i1];
-            cell_st<FAST>(bF, cell_ld<FAST>(bF, cb, r, rowb) + v, cb, r, rowb);
-            if (bF2) cell_st<FAST>(*bF2, cell_ld<FAST>(*bF2, cb, r, rowb) + v, cb, r, rowb);
-        }
+// The fused sources with a corner in the tile at x0, z0 (TZ rows): their
+// wavelet samples, loaded with the tile.  A bit per source in hit.
+struct SrcHits {
+    int hit;
+    float w[kFusedSrc];
+};
+__device__ __forceinline__ SrcHits src_hits(const FusedIO &io, int x0, int z0, int TZ) {
+    SrcHits h;
+    h.hit = 0;
+    for (int i = 0; i < io.nsrc; i++)
+        if (io.sx[i] >= 0 && io.sx[i] + 1 >= x0 && io.sx[i] < x0 + BX && io.sz[i] + 1 >= z0 && io.sz[i] < z0 + TZ)
+            h.hit |= 1 << i;
+#pragma unroll
+    for (int i = 0; i < kFusedSrc; i++) h.w[i] = 0.f;
+    if (h.hit) {
+        const int it = io.it_dev ? *io.it_dev + io.it : io.it;
+#pragma unroll
+        for (int i = 0; i < kFusedSrc; i++)
+            if (i < io.nsrc) h.w[i] = io.wav[(size_t)i * io.src_nt + it];
+    }
+    return h;
+}
+// Injection of the fused sources into a cell (column x, row z) after its
+// stress update: F += (m * w) * xtri * ytri at every source corner, traces in
+// order; m is scale times the modulus.  F2 set: the same term into F2 (elastic
+// explosive source, Sxx and Szz).
+__device__ __forceinline__ void fused_inject(const FusedIO &io, const SrcHits &h, int x, int z, float m, float &F,
+                                             float *F2) {
+#pragma unroll
+    for (int i = 0; i < kFusedSrc; i++) {
+        if (!(h.hit >> i & 1)) continue;
+        const int i1 = z - io.sz[i], i2 = x - io.sx[i];
+        if (i1 < 0 || i1 > 1 || i2 < 0 || i2 > 1) continue;
+        const float v = m * h.w[i] * (i2 ? io.wx[i][1] : io.wx[i][0]) * (i1 ? io.wz[i][1] : io.wz[i][0]);
+        F += v;
+        if (F2) *F2 += v;
     }
 }
 
@@ -186,7 +205,7 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? l
 template <int TZ, int HX, int HZ, bool FAST, class F>
 __device__ __forceinline__ void tile_fetch(Tile<TZ, HX, HZ> &t, F &&ld, int nx, int nz, int x0, int z0) {
     using T = Tile<TZ, HX, HZ>;
-    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int tx = threadIdx.x, ty = block_row();
     const int x = x0 - HX + tx;
     if (FAST) {
         // one VGPR offset; rows k*BZ apart as uniform SGPR offsets
@@ -246,8 +265,35 @@ struct Ld4 {
     }
 };
 
+// Reduced-order differences of an LDS tile, coefficients (ce, the unscaled
+// table) in LDS: a load from memory here would cost its latency per tap.  The
+// taps are the full stencil's; those past order k are not used.
+template <int ORDER>
+__device__ __forceinline__ float dfw_edge(const float *s, int st, const float *ce, int k, float invd) {
+    const float *c = ce + cind(k);
+    float acc = 0.f;
+#pragma unroll
+    for (int io = 0; io < ORDER; io++) acc = io < k ? acc + c[io] * (s[(io + 1) * st] - s[-io * st]) : acc;
+    return acc * invd;
+}
+
 // Derivative of an LDS tile at a cell: compile-time order in the interior,
-// reduced order where the reference's Der shortens the stencil.
+// reduced order where the reference's Der shortens the stencil.  The backward
+// difference is the forward one a cell before.
+template <int ORDER, bool FAST>
+__device__ __forceinline__ float ddfw(const float *s, int st, const float *c, const float *ce, int k, float invd) {
+    float d = dfw<ORDER>(s, st, c + cind(ORDER));
+    if (!FAST && k != ORDER) d = dfw_edge<ORDER>(s, st, ce, k, invd);
+    return d;
+}
+template <int ORDER, bool FAST>
+__device__ __forceinline__ float ddbw(const float *s, int st, const float *c, const float *ce, int k, float invd) {
+    float d = dbw<ORDER>(s, st, c + cind(ORDER));
+    if (!FAST && k != ORDER) d = dfw_edge<ORDER>(s - st, st, ce, k, invd);
+    return d;
+}
+
+// The same with the coefficients in constant memory.
 template <int ORDER, bool FAST>
 __device__ __forceinline__ float ddfw(const float *s, int st, const float *c, int k, float invd) {
     float d = dfw<ORDER>(s, st, c + cind(ORDER));
@@ -293,31 +339,107 @@ __device__ __forceinline__ PmlPos pml_pos(int x, int n, int L) {
     return p;
 }
 
-// Apply dt*M*d then the strip correction of one derivative term.
-template <bool FAST>
-__device__ __forceinline__ void term(float &F, float dtM, float d, const PmlPos &pp, const Tab &tb,
-                                     int stag, float *lo, float *hi, size_t sidx) {
-    F += dtM * d;
-    if (!FAST && pp.side >= 0) {
-        float *psi = (pp.side ? hi : lo) + sidx;
-        pml_corr(F, dtM, psi, tb.A(pp.side, stag, pp.i), tb.B(pp.side, stag, pp.i),
-                 tb.C(pp.side, stag, pp.i), d);
+// A thread's rows against the z strips (uniform) and its column against the x
+// strips; outside both in interior tiles.
+template <int RZ, bool FAST>
+struct Place {
+    PmlPos x, z[RZ];
+    int zt, nx, nz, lpml;
+    __device__ __forceinline__ Place(const K2D &a, int col, int row) : zt(row), nx(a.nx), nz(a.nz), lpml(a.lpml) {
+        x = FAST || col >= nx ? PmlPos{-1, 0} : pml_pos(col, nx, lpml);
+#pragma unroll
+        for (int r = 0; r < RZ; r++) z[r] = FAST || row + r >= nz ? PmlPos{-1, 0} : pml_pos(row + r, nz, lpml);
     }
-}
+};
 
-// The same with the strip's previous value read from ilo / ihi (equal to
-// lo / hi in place).
-template <bool FAST>
-__device__ __forceinline__ void term(float &F, float dtM, float d, const PmlPos &pp, const Tab &tb,
-                                     int stag, float *lo, float *hi, const float *ilo, const float *ihi,
-                                     size_t sidx) {
-    F += dtM * d;
-    if (!FAST && pp.side >= 0) {
-        const float A = tb.A(pp.side, stag, pp.i), B = tb.B(pp.side, stag, pp.i), C = tb.C(pp.side, stag, pp.i);
-        const float p = B * (pp.side ? ihi : ilo)[sidx] + A * d;
-        (pp.side ? hi : lo)[sidx] = p;
-        F -= dtM * (p + C * d);
+// The memory variable of one derivative term at a thread's rows, and its
+// profile values.  load runs with the loads of the tile, without branches: a
+// lane outside the x strips reads some cell of theirs, a row outside the z
+// strips an empty descriptor.  (Loaded where they are used, one term after the
+// other, they cost a boundary tile a memory latency each: us a velocity + a
+// stress step, before -> now, acoustic 190 x 160 order 4 5.6 + 5.7 -> 4.5 +
+// 4.6, order 8 batch of gradient runs 19.3 + 17.4 -> 16.9 + 15.6; elastic
+// 1150 x 920 order 8 22.7 + 26.3 -> 18.2 + 24.2, order 6 on 600 x 470
+// 12.2 + 12.2 -> 8.9 + 10.2.)  step returns psi + C d for psi = B psi + A d
+// (fused in one fixed way, so that every kernel rounds it alike), store writes
+// psi back.
+template <int RZ, bool FAST>
+struct StripX {
+    float A, B, C, v[RZ];
+    float *out;
+    __device__ __forceinline__ void load(const Place<RZ, FAST> &p, const Tab &tb, int stag, const float *ilo,
+                                         const float *ihi, float *lo, float *hi, size_t shot) {
+        if (FAST) return;
+        const int right = p.x.side == 1;
+        A = tb.A(right, stag, p.x.i);
+        B = tb.B(right, stag, p.x.i);
+        C = tb.C(right, stag, p.x.i);
+        const float *in = (right ? ihi : ilo) + shot;
+        out = (right ? hi : lo) + shot + ((size_t)p.zt * p.lpml + p.x.i);
+#pragma unroll
+        for (int r = 0; r < RZ; r++) v[r] = in[(unsigned)(min(p.zt + r, p.nz - 1) * p.lpml + p.x.i)];
     }
+    __device__ __forceinline__ float step(int r, float d) {
+        v[r] = fmaf(A, d, B * v[r]);
+        return v[r] + C * d;
+    }
+    // F += m d and the strip's correction
+    __device__ __forceinline__ void term(const Place<RZ, FAST> &p, float &F, float m, int r, float d) {
+        F += m * d;
+        if (!FAST) {
+            const float q = step(r, d);
+            F = p.x.side >= 0 ? F - m * q : F;
+        }
+    }
+    __device__ __forceinline__ void store(const Place<RZ, FAST> &p, int r) const {
+        if (!FAST && p.x.side >= 0) out[(unsigned)(r * p.lpml)] = v[r];
+    }
+};
+template <int RZ, bool FAST>
+struct StripZ {
+    float A[RZ], B[RZ], C[RZ], v[RZ];
+    float *lo, *hi;
+    __device__ __forceinline__ Buf row(const Place<RZ, FAST> &p, int r, const float *l, const float *h) const {
+        return mkbuf((p.z[r].side == 1 ? h : l) + (size_t)p.z[r].i * p.nx, p.z[r].side >= 0 ? (unsigned)(p.nx * 4) : 0u);
+    }
+    __device__ __forceinline__ void load(const Place<RZ, FAST> &p, const Tab &tb, int stag, const float *ilo,
+                                         const float *ihi, float *l, float *h, size_t shot, int x) {
+        if (FAST) return;
+        lo = l + shot;
+        hi = h + shot;
+#pragma unroll
+        for (int r = 0; r < RZ; r++) {
+            const int right = p.z[r].side == 1, i = p.z[r].i;
+            A[r] = tb.A(right, stag, i);
+            B[r] = tb.B(right, stag, i);
+            C[r] = tb.C(right, stag, i);
+            v[r] = row(p, r, ilo + shot, ihi + shot).ld((unsigned)(x * 4), 0);
+        }
+    }
+    __device__ __forceinline__ float step(int r, float d) {
+        v[r] = fmaf(A[r], d, B[r] * v[r]);
+        return v[r] + C[r] * d;
+    }
+    __device__ __forceinline__ void term(const Place<RZ, FAST> &p, float &F, float m, int r, float d) {
+        F += m * d;
+        if (!FAST && p.z[r].side >= 0) F -= m * step(r, d);
+    }
+    __device__ __forceinline__ void store(const Place<RZ, FAST> &p, int r, int x) const {
+        if (!FAST && p.z[r].side >= 0) row(p, r, lo, hi).st(v[r], (unsigned)(x * 4), 0);
+    }
+};
+
+// Boundary tiles read reduced-order coefficients from LDS: the table, loaded
+// with the tile.
+template <bool FAST>
+__device__ __forceinline__ float edge_fetch() {
+    const int i = threadIdx.x + threadIdx.y * BX;
+    return !FAST && i < 36 ? kCoefC[i] : 0.f;
+}
+template <bool FAST>
+__device__ __forceinline__ void edge_store(float v, float *ce) {
+    const int i = threadIdx.x + threadIdx.y * BX;
+    if (!FAST && i < 36) ce[i] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -327,15 +449,15 @@ __device__ __forceinline__ void term(float &F, float dtM, float d, const PmlPos 
 // Kernel bodies take the LDS buffers from the kernel so the interior (FAST)
 // and boundary instantiations share one allocation.
 template <int ORDER, int RZ, bool FAST>
-__device__ __forceinline__ void a2d_velocity_body(const K2D &a, int x0, int z0, float *sP) {
+__device__ __forceinline__ void a2d_velocity_body(const K2D &a, int x0, int z0, float *sP, float *ce) {
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
-    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = threadIdx.y, x = x0 + tx;
+    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = block_row(), x = x0 + tx, zt = z0 + ty * RZ;
     const bool xin = FAST || x < nx;
     const size_t fo = blockIdx.y * (size_t)a.sf, xo = blockIdx.y * (size_t)a.sxs,
                  zo = blockIdx.y * (size_t)a.szs;
     const unsigned nb = (unsigned)(nx * nz * 4);
     const int rowb = nx * 4;
-    const unsigned cb = (unsigned)(((z0 + ty * RZ) * nx + x) * 4);
+    const unsigned cb = (unsigned)((zt * nx + x) * 4);
     const Buf bVx = mkbuf(a.Vx + fo, nb), bVz = mkbuf(a.Vz + fo, nb), bRx = mkbuf(a.Rx, nb),
               bRz = mkbuf(a.Rz, nb);
     const Buf iVx = mkbuf(a.iVx + fo, nb), iVz = mkbuf(a.iVz + fo, nb);
@@ -347,30 +469,33 @@ __device__ __forceinline__ void a2d_velocity_body(const K2D &a, int x0, int z0, 
         rx[r] = cell_ld<FAST>(bRx, cb, r, rowb);
         rz[r] = cell_ld<FAST>(bRz, cb, r, rowb);
     }
+    const Tab tb{a.tab, a.lpml};
+    const Place<RZ, FAST> pl(a, x, zt);
+    StripX<RZ, FAST> px;
+    StripZ<RZ, FAST> pz;
+    px.load(pl, tb, 1, a.ipsi[RSG_A2D_P_LEFT], a.ipsi[RSG_A2D_P_RIGHT], a.psi[RSG_A2D_P_LEFT], a.psi[RSG_A2D_P_RIGHT], xo);
+    pz.load(pl, tb, 1, a.ipsi[RSG_A2D_P_TOP], a.ipsi[RSG_A2D_P_BOTTOM], a.psi[RSG_A2D_P_TOP], a.psi[RSG_A2D_P_BOTTOM], zo, x);
+    const float cev = edge_fetch<FAST>();
     Tile<TZ, H, H> tp;
     tile_fetch<TZ, H, H, FAST>(tp, Ld1{mkbuf(a.iP + fo, nb)}, nx, nz, x0, z0);
+    edge_store<FAST>(cev, ce);
     tile_store(tp, sP);
     __syncthreads();
     if (!xin) return;
-    const Tab tb{a.tab, a.lpml};
-    const PmlPos px = FAST ? PmlPos{-1, 0} : pml_pos(x, nx, a.lpml);
     const int kx = FAST ? ORDER : kfw(x, nx, ORDER);
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         const int zl = ty * RZ + r, z = z0 + zl;
         if (!FAST && z >= nz) break;
         const float *s = sP + (zl + H) * LD + tx + H;
-        const float dPx = ddfw<ORDER, FAST>(s, 1, a.cx.c, kx, a.invdx);
-        const float dPz = ddfw<ORDER, FAST>(s, LD, a.cz.c, FAST ? ORDER : kfw(z, nz, ORDER), a.invdz);
-        const PmlPos pz = FAST ? PmlPos{-1, 0} : pml_pos(z, nz, a.lpml);
-        term<FAST>(vx[r], a.dt * rx[r], dPx, px, tb, 1, (a.psi[RSG_A2D_P_LEFT] + xo),
-                   (a.psi[RSG_A2D_P_RIGHT] + xo), (a.ipsi[RSG_A2D_P_LEFT] + xo), (a.ipsi[RSG_A2D_P_RIGHT] + xo),
-                   (size_t)z * a.lpml + px.i);
-        term<FAST>(vz[r], a.dt * rz[r], dPz, pz, tb, 1, (a.psi[RSG_A2D_P_TOP] + zo),
-                   (a.psi[RSG_A2D_P_BOTTOM] + zo), (a.ipsi[RSG_A2D_P_TOP] + zo), (a.ipsi[RSG_A2D_P_BOTTOM] + zo),
-                   (size_t)pz.i * nx + x);
+        const float dPx = ddfw<ORDER, FAST>(s, 1, a.cx.c, ce, kx, a.invdx);
+        const float dPz = ddfw<ORDER, FAST>(s, LD, a.cz.c, ce, FAST ? ORDER : kfw(z, nz, ORDER), a.invdz);
+        px.term(pl, vx[r], a.dt * rx[r], r, dPx);
+        pz.term(pl, vz[r], a.dt * rz[r], r, dPz);
         cell_st<FAST>(bVx, vx[r], cb, r, rowb);
         cell_st<FAST>(bVz, vz[r], cb, r, rowb);
+        px.store(pl, r);
+        pz.store(pl, r, x);
     }
 }
 
@@ -378,24 +503,25 @@ template <int ORDER, int RZ>
 __global__ __launch_bounds__(BX *BZ) void a2d_velocity_kernel(const K2D a) {
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
     __shared__ float sP[(TZ + 2 * H) * LD];
+    __shared__ float ce[36];
     int x0, z0;
     if (!tile_of(a, TZ, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        a2d_velocity_body<ORDER, RZ, true>(a, x0, z0, sP);
+        a2d_velocity_body<ORDER, RZ, true>(a, x0, z0, sP, ce);
     else
-        a2d_velocity_body<ORDER, RZ, false>(a, x0, z0, sP);
+        a2d_velocity_body<ORDER, RZ, false>(a, x0, z0, sP, ce);
 }
 
 template <int ORDER, int RZ, bool FAST, bool IO = true>
-__device__ __forceinline__ void a2d_stress_body(const K2D &a, int x0, int z0, float *sVx, float *sVz) {
+__device__ __forceinline__ void a2d_stress_body(const K2D &a, int x0, int z0, float *sVx, float *sVz, float *ce) {
     constexpr int H = ORDER, LDX = BX + 2 * H, LDZ = BX, TZ = BZ * RZ;
-    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = threadIdx.y, x = x0 + tx;
+    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = block_row(), x = x0 + tx, zt = z0 + ty * RZ;
     const bool xin = FAST || x < nx;
     const size_t fo = blockIdx.y * (size_t)a.sf, xo = blockIdx.y * (size_t)a.sxs,
                  zo = blockIdx.y * (size_t)a.szs;
     const unsigned nb = (unsigned)(nx * nz * 4);
     const int rowb = nx * 4;
-    const unsigned cb = (unsigned)(((z0 + ty * RZ) * nx + x) * 4);
+    const unsigned cb = (unsigned)((zt * nx + x) * 4);
     const Buf bP = mkbuf(a.P + fo, nb), bL = mkbuf(a.L, nb), iP = mkbuf(a.iP + fo, nb);
     float pv[RZ], lv[RZ];
 #pragma unroll
@@ -403,34 +529,42 @@ __device__ __forceinline__ void a2d_stress_body(const K2D &a, int x0, int z0, fl
         pv[r] = cell_ld<FAST>(iP, cb, r, rowb);
         lv[r] = cell_ld<FAST>(bL, cb, r, rowb);
     }
+    const Tab tb{a.tab, a.lpml};
+    const Place<RZ, FAST> pl(a, x, zt);
+    StripX<RZ, FAST> px;
+    StripZ<RZ, FAST> pz;
+    px.load(pl, tb, 0, a.ipsi[RSG_A2D_VXX_LEFT], a.ipsi[RSG_A2D_VXX_RIGHT], a.psi[RSG_A2D_VXX_LEFT],
+            a.psi[RSG_A2D_VXX_RIGHT], xo);
+    pz.load(pl, tb, 0, a.ipsi[RSG_A2D_VZZ_TOP], a.ipsi[RSG_A2D_VZZ_BOTTOM], a.psi[RSG_A2D_VZZ_TOP],
+            a.psi[RSG_A2D_VZZ_BOTTOM], zo, x);
+    const float cev = edge_fetch<FAST>();
     Tile<TZ, H, 0> tvx;
     Tile<TZ, 0, H> tvz;
     tile_fetch<TZ, H, 0, FAST>(tvx, Ld1{mkbuf(a.Vx + fo, nb)}, nx, nz, x0, z0);
     tile_fetch<TZ, 0, H, FAST>(tvz, Ld1{mkbuf(a.Vz + fo, nb)}, nx, nz, x0, z0);
+    SrcHits sh;
+    if (IO) sh = src_hits(a.io, x0, z0, TZ);
+    edge_store<FAST>(cev, ce);
     tile_store(tvx, sVx);
     tile_store(tvz, sVz);
     __syncthreads();
     if (!xin) return;
-    const int it = (IO && a.io.nsrc) ? (a.io.it_dev ? *a.io.it_dev + a.io.it : a.io.it) : 0;
-    const Tab tb{a.tab, a.lpml};
-    const PmlPos px = FAST ? PmlPos{-1, 0} : pml_pos(x, nx, a.lpml);
     const int kx = FAST ? ORDER : kbw(x, nx, ORDER);
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         const int zl = ty * RZ + r, z = z0 + zl;
         if (!FAST && z >= nz) break;
-        const float dVx = ddbw<ORDER, FAST>(sVx + zl * LDX + tx + H, 1, a.cx.c, kx, a.invdx);
-        const float dVz = ddbw<ORDER, FAST>(sVz + (zl + H) * LDZ + tx, LDZ, a.cz.c,
+        const float dVx = ddbw<ORDER, FAST>(sVx + zl * LDX + tx + H, 1, a.cx.c, ce, kx, a.invdx);
+        const float dVz = ddbw<ORDER, FAST>(sVz + (zl + H) * LDZ + tx, LDZ, a.cz.c, ce,
                                             FAST ? ORDER : kbw(z, nz, ORDER), a.invdz);
-        const PmlPos pz = FAST ? PmlPos{-1, 0} : pml_pos(z, nz, a.lpml);
         const float dtL = a.dt * lv[r];
-        term<FAST>(pv[r], dtL, dVx, px, tb, 0, (a.psi[RSG_A2D_VXX_LEFT] + xo), (a.psi[RSG_A2D_VXX_RIGHT] + xo),
-                   (a.ipsi[RSG_A2D_VXX_LEFT] + xo), (a.ipsi[RSG_A2D_VXX_RIGHT] + xo), (size_t)z * a.lpml + px.i);
-        term<FAST>(pv[r], dtL, dVz, pz, tb, 0, (a.psi[RSG_A2D_VZZ_TOP] + zo), (a.psi[RSG_A2D_VZZ_BOTTOM] + zo),
-                   (a.ipsi[RSG_A2D_VZZ_TOP] + zo), (a.ipsi[RSG_A2D_VZZ_BOTTOM] + zo), (size_t)pz.i * nx + x);
+        px.term(pl, pv[r], dtL, r, dVx);
+        pz.term(pl, pv[r], dtL, r, dVz);
+        if (IO && sh.hit) fused_inject(a.io, sh, x, z, a.io.scale * lv[r], pv[r], nullptr);
         cell_st<FAST>(bP, pv[r], cb, r, rowb);
+        px.store(pl, r);
+        pz.store(pl, r, x);
     }
-    if (IO && a.io.nsrc) fused_inject<RZ, FAST>(a.io, bP, nullptr, &bL, x, z0 + ty * RZ, nz, cb, rowb, it);
 }
 
 template <int ORDER, int RZ>
@@ -438,12 +572,13 @@ __global__ __launch_bounds__(BX *BZ) void a2d_stress_kernel(const K2D a) {
     constexpr int H = ORDER, TZ = BZ * RZ, LDX = BX + 2 * H, LDZ = BX;
     __shared__ float sVx[TZ * LDX];
     __shared__ float sVz[(TZ + 2 * H) * LDZ];
+    __shared__ float ce[36];
     int x0, z0;
     if (!tile_of(a, TZ, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        a2d_stress_body<ORDER, RZ, true>(a, x0, z0, sVx, sVz);
+        a2d_stress_body<ORDER, RZ, true>(a, x0, z0, sVx, sVz, ce);
     else
-        a2d_stress_body<ORDER, RZ, false>(a, x0, z0, sVx, sVz);
+        a2d_stress_body<ORDER, RZ, false>(a, x0, z0, sVx, sVz, ce);
 }
 
 // ---------------------------------------------------------------------------
@@ -457,16 +592,16 @@ __global__ __launch_bounds__(BX *BZ) void a2d_stress_kernel(const K2D a) {
 // Wzz=L*Sxx+L2M*Szz (adjoint state, waves.cpp:1771-1878).
 template <int ORDER, int RZ, bool BW, bool FAST>
 __device__ __forceinline__ void e2d_velocity_body(const K2D &a, int x0, int z0, float *sXX,
-                                                  float *sZZ, float *sXZ) {
+                                                  float *sZZ, float *sXZ, float *ce) {
     constexpr int H = ORDER, TZ = BZ * RZ;
     constexpr int LDXX = BX + 2 * H, LDZZ = BX, LDXZ = BX + 2 * H;
-    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = threadIdx.y, x = x0 + tx;
+    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = block_row(), x = x0 + tx, zt = z0 + ty * RZ;
     const bool xin = FAST || x < nx;
     const size_t fo = blockIdx.y * (size_t)a.sf, xo = blockIdx.y * (size_t)a.sxs,
                  zo = blockIdx.y * (size_t)a.szs;
     const unsigned nb = (unsigned)(nx * nz * 4);
     const int rowb = nx * 4;
-    const unsigned cb = (unsigned)(((z0 + ty * RZ) * nx + x) * 4);
+    const unsigned cb = (unsigned)((zt * nx + x) * 4);
     const Buf bVx = mkbuf(a.Vx + fo, nb), bVz = mkbuf(a.Vz + fo, nb), bRx = mkbuf(a.Rx, nb),
               bRz = mkbuf(a.Rz, nb);
     float vx[RZ], vz[RZ], rx[RZ], rz[RZ];
@@ -477,6 +612,16 @@ __device__ __forceinline__ void e2d_velocity_body(const K2D &a, int x0, int z0, 
         rx[r] = cell_ld<FAST>(bRx, cb, r, rowb);
         rz[r] = cell_ld<FAST>(bRz, cb, r, rowb);
     }
+    const Tab tb{a.tab, a.lpml};
+    const Place<RZ, FAST> pl(a, x, zt);
+    StripX<RZ, FAST> pxx, pxz;    // of Sxx and Sxz
+    StripZ<RZ, FAST> pzxz, pzz;   // of Sxz and Szz
+#define PSI_(S, LO, HI) a.psi[RSG_E2D_##S##_##LO], a.psi[RSG_E2D_##S##_##HI], a.psi[RSG_E2D_##S##_##LO], a.psi[RSG_E2D_##S##_##HI]
+    pxx.load(pl, tb, 1, PSI_(SXX, LEFT, RIGHT), xo);
+    pxz.load(pl, tb, 0, PSI_(SXZX, LEFT, RIGHT), xo);
+    pzxz.load(pl, tb, 0, PSI_(SXZZ, TOP, BOTTOM), zo, x);
+    pzz.load(pl, tb, 1, PSI_(SZZ, TOP, BOTTOM), zo, x);
+    const float cev = edge_fetch<FAST>();
     Tile<TZ, H, 0> txx;
     Tile<TZ, 0, H> tzz;
     Tile<TZ, H, H> txz;
@@ -491,37 +636,35 @@ __device__ __forceinline__ void e2d_velocity_body(const K2D &a, int x0, int z0, 
         tile_fetch<TZ, 0, H, FAST>(tzz, Ld4{bL, bSxx, bL2M, bSzz}, nx, nz, x0, z0);
         tile_fetch<TZ, H, H, FAST>(txz, Ld2{bM, bSxz}, nx, nz, x0, z0);
     }
+    edge_store<FAST>(cev, ce);
     tile_store(txx, sXX);
     tile_store(tzz, sZZ);
     tile_store(txz, sXZ);
     __syncthreads();
     if (!xin) return;
-    const Tab tb{a.tab, a.lpml};
-    const PmlPos px = FAST ? PmlPos{-1, 0} : pml_pos(x, nx, a.lpml);
     const int kxf = FAST ? ORDER : kfw(x, nx, ORDER), kxb = FAST ? ORDER : kbw(x, nx, ORDER);
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         const int zl = ty * RZ + r, z = z0 + zl;
         if (!FAST && z >= nz) break;
-        const float dSxx = ddfw<ORDER, FAST>(sXX + zl * LDXX + tx + H, 1, a.cx.c, kxf, a.invdx);
+        const int kzf = FAST ? ORDER : kfw(z, nz, ORDER), kzb = FAST ? ORDER : kbw(z, nz, ORDER);
+        const float dSxx = ddfw<ORDER, FAST>(sXX + zl * LDXX + tx + H, 1, a.cx.c, ce, kxf, a.invdx);
         const float *sxz = sXZ + (zl + H) * LDXZ + tx + H;
-        const float dSxz_z = ddbw<ORDER, FAST>(sxz, LDXZ, a.cz.c, FAST ? ORDER : kbw(z, nz, ORDER),
-                                               a.invdz);
-        const float dSxz_x = ddbw<ORDER, FAST>(sxz, 1, a.cx.c, kxb, a.invdx);
-        const float dSzz = ddfw<ORDER, FAST>(sZZ + (zl + H) * LDZZ + tx, LDZZ, a.cz.c,
-                                             FAST ? ORDER : kfw(z, nz, ORDER), a.invdz);
-        const PmlPos pz = FAST ? PmlPos{-1, 0} : pml_pos(z, nz, a.lpml);
-        const size_t ix = (size_t)z * a.lpml + px.i, iz = (size_t)pz.i * nx + x;
+        const float dSxz_z = ddbw<ORDER, FAST>(sxz, LDXZ, a.cz.c, ce, kzb, a.invdz);
+        const float dSxz_x = ddbw<ORDER, FAST>(sxz, 1, a.cx.c, ce, kxb, a.invdx);
+        const float dSzz = ddfw<ORDER, FAST>(sZZ + (zl + H) * LDZZ + tx, LDZZ, a.cz.c, ce, kzf, a.invdz);
         const float dtRx = a.dt * rx[r];
-        term<FAST>(vx[r], dtRx, dSxx, px, tb, 1, (a.psi[RSG_E2D_SXX_LEFT] + xo), (a.psi[RSG_E2D_SXX_RIGHT] + xo), ix);
-        term<FAST>(vx[r], dtRx, dSxz_z, pz, tb, 0, (a.psi[RSG_E2D_SXZZ_TOP] + zo),
-                   (a.psi[RSG_E2D_SXZZ_BOTTOM] + zo), iz);
+        pxx.term(pl, vx[r], dtRx, r, dSxx);
+        pzxz.term(pl, vx[r], dtRx, r, dSxz_z);
         cell_st<FAST>(bVx, vx[r], cb, r, rowb);
         const float dtRz = a.dt * rz[r];
-        term<FAST>(vz[r], dtRz, dSxz_x, px, tb, 0, (a.psi[RSG_E2D_SXZX_LEFT] + xo),
-                   (a.psi[RSG_E2D_SXZX_RIGHT] + xo), ix);
-        term<FAST>(vz[r], dtRz, dSzz, pz, tb, 1, (a.psi[RSG_E2D_SZZ_TOP] + zo), (a.psi[RSG_E2D_SZZ_BOTTOM] + zo), iz);
+        pxz.term(pl, vz[r], dtRz, r, dSxz_x);
+        pzz.term(pl, vz[r], dtRz, r, dSzz);
         cell_st<FAST>(bVz, vz[r], cb, r, rowb);
+        pxx.store(pl, r);
+        pxz.store(pl, r);
+        pzxz.store(pl, r, x);
+        pzz.store(pl, r, x);
     }
 }
 
@@ -531,12 +674,13 @@ __global__ __launch_bounds__(BX *BZ) void e2d_velocity_kernel(const K2D a) {
     __shared__ float sXX[TZ * (BX + 2 * H)];
     __shared__ float sZZ[(TZ + 2 * H) * BX];
     __shared__ float sXZ[(TZ + 2 * H) * (BX + 2 * H)];
+    __shared__ float ce[36];
     int x0, z0;
     if (!tile_of(a, TZ, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        e2d_velocity_body<ORDER, RZ, BW, true>(a, x0, z0, sXX, sZZ, sXZ);
+        e2d_velocity_body<ORDER, RZ, BW, true>(a, x0, z0, sXX, sZZ, sXZ, ce);
     else
-        e2d_velocity_body<ORDER, RZ, BW, false>(a, x0, z0, sXX, sZZ, sXZ);
+        e2d_velocity_body<ORDER, RZ, BW, false>(a, x0, z0, sXX, sZZ, sXZ, ce);
 }
 
 // Stress update.  Forward (BW=false, waves.cpp:1571-1735):
@@ -545,15 +689,15 @@ __global__ __launch_bounds__(BX *BZ) void e2d_velocity_kernel(const K2D a) {
 // Adjoint state (BW=true, waves.cpp:1907-2080): the same derivatives with
 // unit moduli, Sxx only from ddx_bw(Vx) and Szz only from ddz_bw(Vz).
 template <int ORDER, int RZ, bool BW, bool FAST, bool IO = true>
-__device__ __forceinline__ void e2d_stress_body(const K2D &a, int x0, int z0, float *sVx, float *sVz) {
+__device__ __forceinline__ void e2d_stress_body(const K2D &a, int x0, int z0, float *sVx, float *sVz, float *ce) {
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
-    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = threadIdx.y, x = x0 + tx;
+    const int nx = a.nx, nz = a.nz, tx = threadIdx.x, ty = block_row(), x = x0 + tx, zt = z0 + ty * RZ;
     const bool xin = FAST || x < nx;
     const size_t fo = blockIdx.y * (size_t)a.sf, xo = blockIdx.y * (size_t)a.sxs,
                  zo = blockIdx.y * (size_t)a.szs;
     const unsigned nb = (unsigned)(nx * nz * 4);
     const int rowb = nx * 4;
-    const unsigned cb = (unsigned)(((z0 + ty * RZ) * nx + x) * 4);
+    const unsigned cb = (unsigned)((zt * nx + x) * 4);
     const Buf bSxx = mkbuf(a.Sxx + fo, nb), bSzz = mkbuf(a.Szz + fo, nb), bSxz = mkbuf(a.Sxz + fo, nb);
     float sxx[RZ], szz[RZ], sxz[RZ], ml[RZ], ml2m[RZ], mm[RZ];
 #pragma unroll
@@ -567,18 +711,30 @@ __device__ __forceinline__ void e2d_stress_body(const K2D &a, int x0, int z0, fl
             mm[r] = cell_ld<FAST>(mkbuf(a.M, nb), cb, r, rowb);
         }
     }
+    const Tab tb{a.tab, a.lpml};
+    const Place<RZ, FAST> pl(a, x, zt);
+    StripX<RZ, FAST> pxx, pzx;  // of Vx and Vz
+    StripZ<RZ, FAST> pzz, pxz;  // of Vz and Vx
+    pxx.load(pl, tb, 0, PSI_(VXX, LEFT, RIGHT), xo);
+    pzx.load(pl, tb, 1, PSI_(VZX, LEFT, RIGHT), xo);
+    pzz.load(pl, tb, 0, PSI_(VZZ, TOP, BOTTOM), zo, x);
+    pxz.load(pl, tb, 1, PSI_(VXZ, TOP, BOTTOM), zo, x);
+#undef PSI_
+    const float cev = edge_fetch<FAST>();
     Tile<TZ, H, H> tvx, tvz;
     tile_fetch<TZ, H, H, FAST>(tvx, Ld1{mkbuf(a.Vx + fo, nb)}, nx, nz, x0, z0);
     tile_fetch<TZ, H, H, FAST>(tvz, Ld1{mkbuf(a.Vz + fo, nb)}, nx, nz, x0, z0);
+    SrcHits sh;
+    if (IO && !BW) sh = src_hits(a.io, x0, z0, TZ);
+    edge_store<FAST>(cev, ce);
     tile_store(tvx, sVx);
     tile_store(tvz, sVz);
     __syncthreads();
-    const int it = (IO && (a.io.nsrc || a.io.nrec)) ? (a.io.it_dev ? *a.io.it_dev + a.io.it : a.io.it) : 0;
-    if (IO && !BW && a.io.nrec)
+    if (IO && !BW && a.io.nrec) {
+        const int it = a.io.it_dev ? *a.io.it_dev + a.io.it : a.io.it;
         fused_record(a.io, (z0 / TZ) * a.ntx + x0 / BX, x0, z0, H, LD, a.lpml, sVx, sVz, it);
+    }
     if (!xin) return;
-    const Tab tb{a.tab, a.lpml};
-    const PmlPos px = FAST ? PmlPos{-1, 0} : pml_pos(x, nx, a.lpml);
     const int kxf = FAST ? ORDER : kfw(x, nx, ORDER), kxb = FAST ? ORDER : kbw(x, nx, ORDER);
     const float dt = a.dt;
 #pragma unroll
@@ -588,54 +744,48 @@ __device__ __forceinline__ void e2d_stress_body(const K2D &a, int x0, int z0, fl
         const float *svx = sVx + (zl + H) * LD + tx + H;
         const float *svz = sVz + (zl + H) * LD + tx + H;
         const int kzf = FAST ? ORDER : kfw(z, nz, ORDER), kzb = FAST ? ORDER : kbw(z, nz, ORDER);
-        const float dVx_x = ddbw<ORDER, FAST>(svx, 1, a.cx.c, kxb, a.invdx);
-        const float dVz_z = ddbw<ORDER, FAST>(svz, LD, a.cz.c, kzb, a.invdz);
-        const float dVz_x = ddfw<ORDER, FAST>(svz, 1, a.cx.c, kxf, a.invdx);
-        const float dVx_z = ddfw<ORDER, FAST>(svx, LD, a.cz.c, kzf, a.invdz);
-        const PmlPos pz = FAST ? PmlPos{-1, 0} : pml_pos(z, nz, a.lpml);
-        const size_t ix = (size_t)z * a.lpml + px.i, iz = (size_t)pz.i * nx + x;
+        const float dVx_x = ddbw<ORDER, FAST>(svx, 1, a.cx.c, ce, kxb, a.invdx);
+        const float dVz_z = ddbw<ORDER, FAST>(svz, LD, a.cz.c, ce, kzb, a.invdz);
+        const float dVz_x = ddfw<ORDER, FAST>(svz, 1, a.cx.c, ce, kxf, a.invdx);
+        const float dVx_z = ddfw<ORDER, FAST>(svx, LD, a.cz.c, ce, kzf, a.invdz);
         if (!BW) {
             const float dtL2M = dt * ml2m[r], dtL = dt * ml[r];
             // d/dx Vx feeds Sxx (L2M) and Szz (L) through one memory variable
             sxx[r] += dtL2M * dVx_x;
             szz[r] += dtL * dVx_x;
-            if (!FAST && px.side >= 0) {
-                float *psi = a.psi[px.side ? RSG_E2D_VXX_RIGHT : RSG_E2D_VXX_LEFT] + xo + ix;
-                const float A = tb.A(px.side, 0, px.i), B = tb.B(px.side, 0, px.i),
-                            C = tb.C(px.side, 0, px.i);
-                const float q = B * (*psi) + A * dVx_x;
-                *psi = q;
-                sxx[r] -= dtL2M * (q + C * dVx_x);
-                szz[r] -= dtL * (q + C * dVx_x);
+            if (!FAST) {
+                const float q = pxx.step(r, dVx_x);
+                sxx[r] = pl.x.side >= 0 ? sxx[r] - dtL2M * q : sxx[r];
+                szz[r] = pl.x.side >= 0 ? szz[r] - dtL * q : szz[r];
             }
             sxx[r] += dtL * dVz_z;
             szz[r] += dtL2M * dVz_z;
-            if (!FAST && pz.side >= 0) {
-                float *psi = a.psi[pz.side ? RSG_E2D_VZZ_BOTTOM : RSG_E2D_VZZ_TOP] + zo + iz;
-                const float A = tb.A(pz.side, 0, pz.i), B = tb.B(pz.side, 0, pz.i),
-                            C = tb.C(pz.side, 0, pz.i);
-                const float q = B * (*psi) + A * dVz_z;
-                *psi = q;
-                sxx[r] -= dtL * (q + C * dVz_z);
-                szz[r] -= dtL2M * (q + C * dVz_z);
+            if (!FAST && pl.z[r].side >= 0) {
+                const float q = pzz.step(r, dVz_z);
+                sxx[r] -= dtL * q;
+                szz[r] -= dtL2M * q;
             }
             if (!FAST && a.fs && z == a.lpml) szz[r] = 0.f;
             const float dtM = dt * mm[r];
-            term<FAST>(sxz[r], dtM, dVz_x, px, tb, 1, (a.psi[RSG_E2D_VZX_LEFT] + xo), (a.psi[RSG_E2D_VZX_RIGHT] + xo), ix);
-            term<FAST>(sxz[r], dtM, dVx_z, pz, tb, 1, (a.psi[RSG_E2D_VXZ_TOP] + zo), (a.psi[RSG_E2D_VXZ_BOTTOM] + zo), iz);
+            pzx.term(pl, sxz[r], dtM, r, dVz_x);
+            pxz.term(pl, sxz[r], dtM, r, dVx_z);
+            // explosive source: Sxx, Szz -= dt * w * xtri * ytri
+            if (IO && sh.hit) fused_inject(a.io, sh, x, z, a.io.scale, sxx[r], &szz[r]);
         } else {
-            term<FAST>(sxx[r], dt, dVx_x, px, tb, 0, (a.psi[RSG_E2D_VXX_LEFT] + xo), (a.psi[RSG_E2D_VXX_RIGHT] + xo), ix);
-            term<FAST>(szz[r], dt, dVz_z, pz, tb, 0, (a.psi[RSG_E2D_VZZ_TOP] + zo), (a.psi[RSG_E2D_VZZ_BOTTOM] + zo), iz);
+            pxx.term(pl, sxx[r], dt, r, dVx_x);
+            pzz.term(pl, szz[r], dt, r, dVz_z);
             if (!FAST && a.fs && z == a.lpml) szz[r] = 0.f;
-            term<FAST>(sxz[r], dt, dVz_x, px, tb, 1, (a.psi[RSG_E2D_VZX_LEFT] + xo), (a.psi[RSG_E2D_VZX_RIGHT] + xo), ix);
-            term<FAST>(sxz[r], dt, dVx_z, pz, tb, 1, (a.psi[RSG_E2D_VXZ_TOP] + zo), (a.psi[RSG_E2D_VXZ_BOTTOM] + zo), iz);
+            pzx.term(pl, sxz[r], dt, r, dVz_x);
+            pxz.term(pl, sxz[r], dt, r, dVx_z);
         }
         cell_st<FAST>(bSxx, sxx[r], cb, r, rowb);
         cell_st<FAST>(bSzz, szz[r], cb, r, rowb);
         cell_st<FAST>(bSxz, sxz[r], cb, r, rowb);
+        pxx.store(pl, r);
+        pzx.store(pl, r);
+        pzz.store(pl, r, x);
+        pxz.store(pl, r, x);
     }
-    // explosive source: Sxx, Szz -= dt * w * xtri * ytri
-    if (IO && !BW && a.io.nsrc) fused_inject<RZ, FAST>(a.io, bSxx, &bSzz, nullptr, x, z0 + ty * RZ, nz, cb, rowb, it);
 }
 
 template <int ORDER, int RZ, bool BW>
@@ -643,12 +793,13 @@ __global__ __launch_bounds__(BX *BZ) void e2d_stress_kernel(const K2D a) {
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
     __shared__ float sVx[(TZ + 2 * H) * LD];
     __shared__ float sVz[(TZ + 2 * H) * LD];
+    __shared__ float ce[36];
     int x0, z0;
     if (!tile_of(a, TZ, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        e2d_stress_body<ORDER, RZ, BW, true>(a, x0, z0, sVx, sVz);
+        e2d_stress_body<ORDER, RZ, BW, true>(a, x0, z0, sVx, sVz, ce);
     else
-        e2d_stress_body<ORDER, RZ, BW, false>(a, x0, z0, sVx, sVz);
+        e2d_stress_body<ORDER, RZ, BW, false>(a, x0, z0, sVx, sVz, ce);
 }
 
 // ---------------------------------------------------------------------------
@@ -689,13 +840,14 @@ __global__ __launch_bounds__(BX *BZ) void a2d_velocity_ragged_kernel(const K2D *
                                                                       const int *__restrict__ tile0, int nshot) {
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
     __shared__ float sP[(TZ + 2 * H) * LD];
+    __shared__ float ce[36];
     K2D a;
     int x0, z0;
     if (!ragged_tile(desc, tile0, nshot, TZ, a, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        a2d_velocity_body<ORDER, RZ, true>(a, x0, z0, sP);
+        a2d_velocity_body<ORDER, RZ, true>(a, x0, z0, sP, ce);
     else
-        a2d_velocity_body<ORDER, RZ, false>(a, x0, z0, sP);
+        a2d_velocity_body<ORDER, RZ, false>(a, x0, z0, sP, ce);
 }
 
 template <int ORDER, int RZ>
@@ -704,13 +856,14 @@ __global__ __launch_bounds__(BX *BZ) void a2d_stress_ragged_kernel(const K2D *__
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
     __shared__ float sVx[TZ * LD];
     __shared__ float sVz[(TZ + 2 * H) * BX];
+    __shared__ float ce[36];
     K2D a;
     int x0, z0;
     if (!ragged_tile(desc, tile0, nshot, TZ, a, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        a2d_stress_body<ORDER, RZ, true, false>(a, x0, z0, sVx, sVz);
+        a2d_stress_body<ORDER, RZ, true, false>(a, x0, z0, sVx, sVz, ce);
     else
-        a2d_stress_body<ORDER, RZ, false, false>(a, x0, z0, sVx, sVz);
+        a2d_stress_body<ORDER, RZ, false, false>(a, x0, z0, sVx, sVz, ce);
 }
 
 template <int ORDER, int RZ, bool BW>
@@ -720,13 +873,14 @@ __global__ __launch_bounds__(BX *BZ) void e2d_velocity_ragged_kernel(const K2D *
     __shared__ float sXX[TZ * (BX + 2 * H)];
     __shared__ float sZZ[(TZ + 2 * H) * BX];
     __shared__ float sXZ[(TZ + 2 * H) * (BX + 2 * H)];
+    __shared__ float ce[36];
     K2D a;
     int x0, z0;
     if (!ragged_tile(desc, tile0, nshot, TZ, a, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        e2d_velocity_body<ORDER, RZ, BW, true>(a, x0, z0, sXX, sZZ, sXZ);
+        e2d_velocity_body<ORDER, RZ, BW, true>(a, x0, z0, sXX, sZZ, sXZ, ce);
     else
-        e2d_velocity_body<ORDER, RZ, BW, false>(a, x0, z0, sXX, sZZ, sXZ);
+        e2d_velocity_body<ORDER, RZ, BW, false>(a, x0, z0, sXX, sZZ, sXZ, ce);
 }
 
 template <int ORDER, int RZ, bool BW>
@@ -735,13 +889,14 @@ __global__ __launch_bounds__(BX *BZ) void e2d_stress_ragged_kernel(const K2D *__
     constexpr int H = ORDER, TZ = BZ * RZ, LD = BX + 2 * H;
     __shared__ float sVx[(TZ + 2 * H) * LD];
     __shared__ float sVz[(TZ + 2 * H) * LD];
+    __shared__ float ce[36];
     K2D a;
     int x0, z0;
     if (!ragged_tile(desc, tile0, nshot, TZ, a, x0, z0)) return;
     if (interior_tile(a, x0, z0, TZ, H))
-        e2d_stress_body<ORDER, RZ, BW, true, false>(a, x0, z0, sVx, sVz);
+        e2d_stress_body<ORDER, RZ, BW, true, false>(a, x0, z0, sVx, sVz, ce);
     else
-        e2d_stress_body<ORDER, RZ, BW, false, false>(a, x0, z0, sVx, sVz);
+        e2d_stress_body<ORDER, RZ, BW, false, false>(a, x0, z0, sVx, sVz, ce);
 }
 
 // ---------------------------------------------------------------------------
