@@ -44,20 +44,22 @@ __global__ __launch_bounds__(256) void crosscorr_a3d_kernel(
     const size_t m = ((size_t)iz * ny + iy) * nx + ix;
     const float vpscale = (float)(-2.0 / (double)Vp[m]);
     const float rhoscale1 = (float)(-1.0 / (double)Rho[m]);
-    const float mrxx = (wrx[q] - wrx[q - 1]) / dx;
-    const float mryy = (wry[q] - wry[q - nxp]) / dy;
-    const float mrzz = (wrz[q] - wrz[q - nxyp]) / dz;
+    // x / h as x * (1 / h) in double, rounded to float afterwards: within one
+    // double ulp of the quotient
+    const double idx = 1.0 / (double)dx, idy = 1.0 / (double)dy, idz = 1.0 / (double)dz;
+    auto div = [](float d, double h) { return (float)((double)d * h); };
+    const float mrxx = div(wrx[q] - wrx[q - 1], idx);
+    const float mryy = div(wry[q] - wry[q - nxp], idy);
+    const float mrzz = div(wrz[q] - wrz[q - nxyp], idz);
     const float ws = wsp[q];
     vpgrad[m] -= vpscale * ws * (mrxx + mryy + mrzz);
     float rg = rhograd[m] - rhoscale1 * ws * (mrxx + mryy + mrzz);
-    float ux = (float)(0.5 * (double)wrx[q] * (double)Rx[q] * (double)(wsp[q + 1] - ws) / (double)dx);
-    ux = (float)((double)ux + 0.5 * (double)wrx[q - 1] * (double)Rx[q - 1] * (double)(ws - wsp[q - 1]) / (double)dx);
-    float uy = (float)(0.5 * (double)wry[q] * (double)Ry[q] * (double)(wsp[q + nxp] - ws) / (double)dy);
-    uy = (float)((double)uy + 0.5 * (double)wry[q - nxp] * (double)Ry[q - nxp] * (double)(ws - wsp[q - nxp]) /
-                                  (double)dy);
-    float uz = (float)(0.5 * (double)wrz[q] * (double)Rz[q] * (double)(wsp[q + nxyp] - ws) / (double)dz);
-    uz = (float)((double)uz + 0.5 * (double)wrz[q - nxp] * (double)Rz[q - nxyp] * (double)(ws - wsp[q - nxyp]) /
-                                  (double)dz);
+    float ux = (float)(0.5 * (double)wrx[q] * (double)Rx[q] * (double)(wsp[q + 1] - ws) * idx);
+    ux = (float)((double)ux + 0.5 * (double)wrx[q - 1] * (double)Rx[q - 1] * (double)(ws - wsp[q - 1]) * idx);
+    float uy = (float)(0.5 * (double)wry[q] * (double)Ry[q] * (double)(wsp[q + nxp] - ws) * idy);
+    uy = (float)((double)uy + 0.5 * (double)wry[q - nxp] * (double)Ry[q - nxp] * (double)(ws - wsp[q - nxp]) * idy);
+    float uz = (float)(0.5 * (double)wrz[q] * (double)Rz[q] * (double)(wsp[q + nxyp] - ws) * idz);
+    uz = (float)((double)uz + 0.5 * (double)wrz[q - nxp] * (double)Rz[q - nxyp] * (double)(ws - wsp[q - nxyp]) * idz);
     rhograd[m] = rg + (ux + uy + uz);
 }
 

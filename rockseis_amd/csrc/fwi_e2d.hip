@@ -192,27 +192,35 @@ __global__ __launch_bounds__(256) void e2d_crosscorr_kernel(const ShotDev *__res
     const size_t q = (size_t)(iz + s.lpml) * n + ix + s.lpml;
     const float *wsx = s.fVx, *wsz = s.fVz, *wsxx = s.fSxx, *wszz = s.fSzz, *wsxz = s.fSxz;
     const float *wrx = s.bVx, *wrz = s.bVz, *rsxx = s.bSxx, *rszz = s.bSzz, *rsxz = s.bSxz;
-    const float msxx = (wsx[q] - wsx[q - 1]) / dx;
-    const float mszz = (wsz[q] - wsz[q - n]) / dz;
+    // x / h as x * (1 / h) in double, rounded to float afterwards: within one
+    // double ulp of the quotient (six windows of 1600 x 400: 31.8 -> 30.9 us,
+    // what is left are the 18 arrays)
+    const double idx = 1.0 / (double)dx, idz = 1.0 / (double)dz;
+    auto div = [](float d, double h) { return (float)((double)d * h); };
     const size_t m = (size_t)iz * s.nx + ix;
-    s.lam[m] -= (msxx + mszz) * (rsxx[q] + rszz[q]);
-    const float msxz1 = (wsx[q - 1] - wsx[q - 1 - n]) / dz + (wsz[q - n] - wsz[q - 1 - n]) / dx;
-    const float msxz2 = (wsx[q] - wsx[q - n]) / dz + (wsz[q + 1 - n] - wsz[q - n]) / dx;
-    const float msxz3 = (wsx[q - 1 + n] - wsx[q - 1]) / dz + (wsz[q] - wsz[q - 1]) / dx;
-    const float msxz4 = (wsx[q + n] - wsx[q]) / dz + (wsz[q + 1] - wsz[q]) / dx;
+    const float lam = s.lam[m], mu = s.mu[m], rho = s.rho[m];
+    const float msxx = div(wsx[q] - wsx[q - 1], idx);
+    const float mszz = div(wsz[q] - wsz[q - n], idz);
+    const float dlam = (msxx + mszz) * (rsxx[q] + rszz[q]);
+    const float msxz1 = div(wsx[q - 1] - wsx[q - 1 - n], idz) + div(wsz[q - n] - wsz[q - 1 - n], idx);
+    const float msxz2 = div(wsx[q] - wsx[q - n], idz) + div(wsz[q + 1 - n] - wsz[q - n], idx);
+    const float msxz3 = div(wsx[q - 1 + n] - wsx[q - 1], idz) + div(wsz[q] - wsz[q - 1], idx);
+    const float msxz4 = div(wsx[q + n] - wsx[q], idz) + div(wsz[q + 1] - wsz[q], idx);
     const float f1 = msxx * rszz[q] + mszz * rsxx[q];
     const float f2 = msxz1 * rsxz[q - 1 - n] + msxz2 * rsxz[q - n] + msxz3 * rsxz[q - 1] + msxz4 * rsxz[q];
-    s.mu[m] = (float)((double)s.mu[m] + (2.0 * (double)f1 - 0.25 * (double)f2));
     const double rx0 = s.Rx[q], rx1 = s.Rx[q - 1], rz0 = s.Rz[q], rz1 = s.Rz[q - n];
-    float ux = (float)(0.5 * (double)wrx[q] * rx0 * (double)(wsxx[q + 1] - wsxx[q]) / (double)dx);
-    ux = (float)((double)ux + 0.5 * (double)wrx[q - 1] * rx1 * (double)(wsxx[q] - wsxx[q - 1]) / (double)dx);
-    ux = (float)((double)ux + 0.5 * (double)wrx[q] * rx0 * (double)(wsxz[q] - wsxz[q - n]) / (double)dz);
-    ux = (float)((double)ux + 0.5 * (double)wrx[q - 1] * rx1 * (double)(wsxz[q - 1] - wsxz[q - 1 - n]) / (double)dz);
-    float uz = (float)(0.5 * (double)wrz[q] * rz0 * (double)(wsxz[q] - wsxz[q - 1]) / (double)dx);
-    uz = (float)((double)uz + 0.5 * (double)wrz[q - n] * rz1 * (double)(wsxz[q - n] - wsxz[q - 1 - n]) / (double)dx);
-    uz = (float)((double)uz + 0.5 * (double)wrz[q] * rz0 * (double)(wszz[q + n] - wszz[q]) / (double)dz);
-    uz = (float)((double)uz + 0.5 * (double)wrz[q - n] * rz1 * (double)(wszz[q] - wszz[q - n]) / (double)dz);
-    s.rho[m] -= (ux + uz);
+    float ux = (float)(0.5 * (double)wrx[q] * rx0 * (double)(wsxx[q + 1] - wsxx[q]) * idx);
+    ux = (float)((double)ux + 0.5 * (double)wrx[q - 1] * rx1 * (double)(wsxx[q] - wsxx[q - 1]) * idx);
+    ux = (float)((double)ux + 0.5 * (double)wrx[q] * rx0 * (double)(wsxz[q] - wsxz[q - n]) * idz);
+    ux = (float)((double)ux + 0.5 * (double)wrx[q - 1] * rx1 * (double)(wsxz[q - 1] - wsxz[q - 1 - n]) * idz);
+    float uz = (float)(0.5 * (double)wrz[q] * rz0 * (double)(wsxz[q] - wsxz[q - 1]) * idx);
+    uz = (float)((double)uz + 0.5 * (double)wrz[q - n] * rz1 * (double)(wsxz[q - n] - wsxz[q - 1 - n]) * idx);
+    uz = (float)((double)uz + 0.5 * (double)wrz[q] * rz0 * (double)(wszz[q + n] - wszz[q]) * idz);
+    uz = (float)((double)uz + 0.5 * (double)wrz[q - n] * rz1 * (double)(wszz[q] - wszz[q - n]) * idz);
+    // stored last: the compiler may not move a load above a store
+    s.lam[m] = lam - dlam;
+    s.mu[m] = (float)((double)mu + (2.0 * (double)f1 - 0.25 * (double)f2));
+    s.rho[m] = rho - (ux + uz);
 }
 
 // Stack every window's kernels into the caller's images (x offset ox, z

@@ -357,10 +357,10 @@ struct Place {
 // lane outside the x strips reads some cell of theirs, a row outside the z
 // strips an empty descriptor.  (Loaded where they are used, one term after the
 // other, they cost a boundary tile a memory latency each: us a velocity + a
-// stress step, before -> now, acoustic 190 x 160 order 4 5.6 + 5.7 -> 4.5 +
-// 4.6, order 8 batch of gradient runs 19.3 + 17.4 -> 16.9 + 15.6; elastic
-// 1150 x 920 order 8 22.7 + 26.3 -> 18.2 + 24.2, order 6 on 600 x 470
-// 12.2 + 12.2 -> 8.9 + 10.2.)  step returns psi + C d for psi = B psi + A d
+// stress step, before -> now, acoustic 161 x 137 order 4 5.6 + 5.7 -> 4.5 +
+// 4.6, eight of 861 x 461 order 8 19.3 + 17.4 -> 16.9 + 15.6; elastic 2081 x
+// 1081 order 8 22.7 + 26.3 -> 18.2 + 24.2, 1253 x 567 order 6 12.2 + 12.2 ->
+// 8.9 + 10.2.)  step returns psi + C d for psi = B psi + A d
 // (fused in one fixed way, so that every kernel rounds it alike), store writes
 // psi back.
 template <int RZ, bool FAST>
