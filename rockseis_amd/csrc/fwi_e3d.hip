@@ -380,12 +380,12 @@ static int fwi_e3d_impl(const rsg_grid *g, const rsg_fwi_e3d *f, hipStream_t st)
         case RSG_VZ: F[0] = sf.Vz; M = f->Rz; break;
         default: F[0] = sf.Sxx; F[1] = sf.Syy; F[2] = sf.Szz; scale = -g->dt; break;  // explosive: -dt wav w
         }
-        for (int j = 0; j < 3 && F[j]; j++) {
-            inject3d_ordered_kernel<<<(osrc.ncells + 63) / 64, 64, 0, st>>>(F[j], M, scale, osrc.cells, osrc.starts,
-                                                                            osrc.ents, osrc.ncells, f->src.shift,
-                                                                            f->src.data, nt, it);
-            RSG_LAUNCH_CHECK("inject3d_ordered_kernel");
-        }
+        Injects3D in{};
+        int n = 0;
+        for (; n < 3 && F[n]; n++)
+            in.s[n] = {F[n], M, f->src.shift, f->src.data, osrc.cells, osrc.starts, osrc.ents, osrc.ncells};
+        inject3d_ordered_sets_kernel<<<dim3((osrc.ncells + 63) / 64, n), 64, 0, st>>>(in, scale, nt, it);
+        RSG_LAUNCH_CHECK("inject3d_ordered_sets_kernel");
         return RSG_OK;
     };
     auto fstep = [&](int it, bool rec) -> int {
@@ -403,13 +403,16 @@ static int fwi_e3d_impl(const rsg_grid *g, const rsg_fwi_e3d *f, hipStream_t st)
     auto reverse_tail = [&](int capo) -> int {
         float *F[3] = {sb.Vx, sb.Vy, sb.Vz};
         const float *M[3] = {f->Rx, f->Ry, f->Rz};
-        for (int c = 0; c < 3; c++)
-            if (ores[c].ncells > 0) {
-                inject3d_ordered_kernel<<<(ores[c].ncells + 63) / 64, 64, 0, st>>>(
-                    F[c], M[c], g->dt, ores[c].cells, ores[c].starts, ores[c].ents, ores[c].ncells, f->obs[c].shift,
-                    f->dres[c], nt, capo);
-                RSG_LAUNCH_CHECK("inject3d_ordered_kernel");
-            }
+        Injects3D in{};
+        int most = 0;
+        for (int c = 0; c < 3; c++) {
+            in.s[c] = {F[c], M[c], f->obs[c].shift, f->dres[c], ores[c].cells, ores[c].starts, ores[c].ents, ores[c].ncells};
+            most = std::max(most, (int)ores[c].ncells);
+        }
+        if (most > 0) {
+            inject3d_ordered_sets_kernel<<<dim3((most + 63) / 64, 3), 64, 0, st>>>(in, g->dt, nt, capo);
+            RSG_LAUNCH_CHECK("inject3d_ordered_sets_kernel");
+        }
         if (interior) {
             crosscorr_e3d_kernel<<<xg, xb, 0, st>>>(xc);
             RSG_LAUNCH_CHECK("crosscorr_e3d_kernel");

@@ -171,14 +171,12 @@ struct OrderedInject3D {
     }
 };
 
-// P += dt * L * res * xtri * ytri * ztri (L null: dt * res * ...), cell by
-// cell in trace order.
-__global__ void inject3d_ordered_kernel(float *P, const float *__restrict__ L, float dt,
-                                        const size_t *__restrict__ cells, const int *__restrict__ starts,
-                                        const int *__restrict__ ents, int ncells, const float *__restrict__ shift,
-                                        const float *__restrict__ wav, int nt, int it) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ncells) return;
+// P += dt * L * res * xtri * ytri * ztri (L null: dt * res * ...) at cell j of
+// the list, in trace order.
+__device__ __forceinline__ void inject3d_cell(int j, float *P, const float *__restrict__ L, float dt,
+                                              const size_t *__restrict__ cells, const int *__restrict__ starts,
+                                              const int *__restrict__ ents, const float *__restrict__ shift,
+                                              const float *__restrict__ wav, int nt, int it) {
     const size_t p = cells[j];
     const float m = L ? dt * L[p] : dt;
     float a = P[p];
@@ -189,6 +187,32 @@ __global__ void inject3d_ordered_kernel(float *P, const float *__restrict__ L, f
         a += m * wav[(size_t)i * nt + it] * xt * yt * zt;
     }
     P[p] = a;
+}
+__global__ void inject3d_ordered_kernel(float *P, const float *__restrict__ L, float dt,
+                                        const size_t *__restrict__ cells, const int *__restrict__ starts,
+                                        const int *__restrict__ ents, int ncells, const float *__restrict__ shift,
+                                        const float *__restrict__ wav, int nt, int it) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < ncells) inject3d_cell(j, P, L, dt, cells, starts, ents, shift, wav, nt, it);
+}
+
+// Up to three injections into different fields in one launch (blockIdx.y):
+// each is one latency chain of 4.7 us, side by side they cost one (elastic 3D
+// gradient of a 100 x 90 x 80 model: 681 launches -> 227, 54.9 -> 53.4 ms).
+struct Inject3D {
+    float *P;
+    const float *L, *shift, *wav;
+    const size_t *cells;
+    const int *starts, *ents;
+    int ncells;
+};
+struct Injects3D {
+    Inject3D s[3];
+};
+__global__ void inject3d_ordered_sets_kernel(const Injects3D a, float dt, int nt, int it) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const Inject3D &s = a.s[blockIdx.y];
+    if (j < s.ncells) inject3d_cell(j, s.P, s.L, dt, s.cells, s.starts, s.ents, s.shift, s.wav, nt, it);
 }
 
 }  // namespace
