@@ -5,8 +5,10 @@
 
 namespace rsg {
 
+// The queue, three fields and three moduli are a few registers too many for
+// four waves a SIMD from order 7 on (four spill 16 bytes a lane).
 template <int TX, int ORDER>
-__global__ RSG3_BOUNDS void a3d_velocity_kernel(const G3 g, const Grad3Args a) {
+__global__ __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu((ORDER) >= 7 ? 3 : 4, 8))) void a3d_velocity_kernel(const G3 g, const Grad3Args a) {
     using K = Grad3<TX, ORDER>;
     __shared__ float lds[K::LDS];
     Pos3 p;
