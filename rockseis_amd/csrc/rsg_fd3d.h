@@ -519,7 +519,8 @@ struct Div3 {
                     for (int i = 0; i < NOUT; i++)
                         if (!(NOUT == 3 && UNIT && i != a)) strip3(F[i][r], m(a, i), d, in, C, psi);
                 };
-                if (HX) {
+                auto term_x = [&]() RSG_INLINE {
+                    if (!HX) return;
                     // the backward difference is the forward one a cell before
                     const float *w = bx + yl * WX::LD + ln.tx + H - 1 + fx;
                     float d = dfw<ORDER>(w, 1, g.c[0]);
@@ -527,28 +528,40 @@ struct Div3 {
                         if (sd.kx != H) d = dfw_edge(w, 1, sd.kx, g.inv[0], ce);
                     plain(0, d);
                     if (PXY && sd.px) {
-                        sx[r] = sd.x.B * sx[r] + sd.x.A * d;
+                        sx[r] = fmaf(sd.x.A, d, sd.x.B * sx[r]);
                         strip(0, d, sd.inx[r], sd.x.C, sx[r]);
                     }
-                }
-                if (HY) {
+                };
+                auto term_y = [&]() RSG_INLINE {
+                    if (!HY) return;
                     const float *w = by + (yl + H - 1 + fy) * WY::LD + ln.tx;
                     float d = dfw<ORDER>(w, WY::LD, g.c[1]);
                     if (PXY && sd.ey)
                         if (sd.ky[r] != H) d = dfw_edge(w, WY::LD, sd.ky[r], g.inv[1], ce);
                     plain(1, d);
                     if (PXY && sd.py) {
-                        sy[r] = sd.y[r].B * sy[r] + sd.y[r].A * d;
+                        sy[r] = fmaf(sd.y[r].A, d, sd.y[r].B * sy[r]);
                         strip(1, d, sd.y[r].in, sd.y[r].C, sy[r]);
                     }
-                }
-                if (HZ) {
+                };
+                auto term_z = [&]() RSG_INLINE {
+                    if (!HZ) return;
                     const float d = PZ ? dq_edge<H, sb>(q[r], cz, kz) : dq<H, sb>(q[r], g.c[2]);
                     plain(2, d);
                     if (PZ && zin) {
-                        zv.v[r] = zv.B * zv.v[r] + zv.A * d;
+                        zv.v[r] = fmaf(zv.A, d, zv.B * zv.v[r]);
                         strip(2, d, true, zv.C, zv.v[r]);
                     }
+                };
+                // the reference's order: x, y, z, but z, y for Syz and y, x for Sxy
+                if (HX && HZ) {
+                    term_x();
+                    term_y();
+                    term_z();
+                } else {
+                    term_z();
+                    term_y();
+                    term_x();
                 }
                 // free surface: the plane lpml lies in no z strip, so zeroing
                 // after the strips is the reference's zeroing before them
@@ -663,7 +676,7 @@ struct Grad3 {
                     if (sd.kx != H) d = dfw_edge(t, 1, sd.kx, g.inv[0], ce);
                 V[0][r] += m * d;
                 if (PXY && sd.px) {
-                    sx[r] = sd.x.B * sx[r] + sd.x.A * d;
+                    sx[r] = fmaf(sd.x.A, d, sd.x.B * sx[r]);
                     strip3(V[0][r], m, d, sd.inx[r], sd.x.C, sx[r]);
                 }
                 m = g.dt * R[1][r];
@@ -672,14 +685,14 @@ struct Grad3 {
                     if (sd.ky[r] != H) d = dfw_edge(t, W::LD, sd.ky[r], g.inv[1], ce);
                 V[1][r] += m * d;
                 if (PXY && sd.py) {
-                    sy[r] = sd.y[r].B * sy[r] + sd.y[r].A * d;
+                    sy[r] = fmaf(sd.y[r].A, d, sd.y[r].B * sy[r]);
                     strip3(V[1][r], m, d, sd.y[r].in, sd.y[r].C, sy[r]);
                 }
                 m = g.dt * R[2][r];
                 d = PZ ? dq_edge<H, sb>(q[r], cz, kz) : dq<H, sb>(q[r], g.c[2]);
                 V[2][r] += m * d;
                 if (PZ && zin) {
-                    zv.v[r] = zv.B * zv.v[r] + zv.A * d;
+                    zv.v[r] = fmaf(zv.A, d, zv.B * zv.v[r]);
                     strip3(V[2][r], m, d, true, zv.C, zv.v[r]);
                 }
             }
