@@ -303,7 +303,8 @@ typedef struct {
 int rsg_stagger_e3d(const float *vp, const float *vs, const float *rho, int nx, int ny, int nz, int lpml, int fs,
                     float *L, float *L2M, float *Mxz, float *Myz, float *Mxy, float *Rx, float *Ry, float *Rz);
 /* forwardstepVelocity / forwardstepStress (waves.cpp:2465-3258); g: padded
- * sizes (2 lpml < n, nz <= 65535), fs zeroes Szz on plane lpml. */
+ * sizes (2 lpml < n, nz <= 65535, nx min(ny, 8 + 2 order) < 2^30), fs zeroes
+ * Szz on plane lpml. */
 int rsg_e3d_forward_velocity(const rsg_grid *g, const rsg_state_e3d *s, void *stream);
 int rsg_e3d_forward_stress(const rsg_grid *g, const rsg_state_e3d *s, void *stream);
 /* insertSource (waves.cpp:4104-4246): PRESSURE explosive into Sxx, Syy,

@@ -269,8 +269,6 @@ int check_e3d(const rsg_grid *g, const rsg_state_e3d *s) {
     if (g->nx < 2 || g->ny < 2 || g->nz < 2 || g->nz > 65535 || g->lpml < 1 || 2 * g->lpml >= g->nx ||
         2 * g->lpml >= g->ny || 2 * g->lpml >= g->nz || g->dx <= 0 || g->dy <= 0 || g->dz <= 0)
         return fail(RSG_EINVAL, "e3d: grid sizes (padded, 2 lpml < n, nz <= 65535) or steps");
-    if (g->nx >= 1 << 24 && (long long)g->nx * g->ny * 4 >= (1LL << 31))
-        return fail(RSG_EINVAL, "e3d: a tile's rows exceed 32-bit offsets (nx >= 2^24 and plane >= 2^29 cells)");
     if (!s->Vx || !s->Vy || !s->Vz || !s->Sxx || !s->Syy || !s->Szz || !s->Syz || !s->Sxz || !s->Sxy || !s->L ||
         !s->L2M || !s->Mxz || !s->Myz || !s->Mxy || !s->Rx || !s->Ry || !s->Rz || !s->tab)
         return fail(RSG_EINVAL, "e3d: null field, model or table");
@@ -358,6 +356,7 @@ namespace rsg {
 // stresses once per cell, then the forward velocity step on them.
 int e3d_backward_velocity_premul(const rsg_grid *g, const rsg_state_e3d *s, float *scratch, hipStream_t st) {
     if (int rc = check_e3d(g, s)) return rc;
+    if (int rc = check_tiles3(g)) return rc;
     if (!scratch) return fail(RSG_EINVAL, "e3d: null scratch");
     const K3E k = make_k3e(g, s);
     const size_t n = (size_t)g->nx * g->ny * g->nz;
@@ -374,11 +373,13 @@ extern "C" {
 
 int rsg_e3d_forward_velocity(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
     if (int rc = rsg::check_e3d(g, s)) return rc;
+    if (int rc = rsg::check_tiles3(g)) return rc;
     return rsg::launch_velocity(g, s, s->Sxx, s->Syy, s->Szz, s->Syz, s->Sxz, s->Sxy, (hipStream_t)stream);
 }
 
 int rsg_e3d_forward_stress(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
     if (int rc = rsg::check_e3d(g, s)) return rc;
+    if (int rc = rsg::check_tiles3(g)) return rc;
     return rsg::e3d_stress_forward(g, s, (hipStream_t)stream);
 }
 
@@ -399,6 +400,7 @@ int rsg_e3d_backward_velocity_ws(const rsg_grid *g, const rsg_state_e3d *s, floa
 
 int rsg_e3d_backward_stress(const rsg_grid *g, const rsg_state_e3d *s, void *stream) {
     if (int rc = rsg::check_e3d(g, s)) return rc;
+    if (int rc = rsg::check_tiles3(g)) return rc;
     return rsg::e3d_stress_backward(g, s, (hipStream_t)stream);
 }
 

@@ -17,6 +17,15 @@ struct Comps3 {
 inline Term3 term(const float *f, const rsg_state_e3d *s, int slot, int fw) {
     return Term3{f, s->psi[slot], s->psi[slot + 1], fw};
 }
+// The elastic steps take planes of any size (the acoustic ones up to 2^29
+// cells, whose offsets always fit): those whose windows reach past 32-bit
+// offsets, a row's cells times the window's rows (8 + 2 order, or ny) from 2^30
+// on, are left to no kernel.  Rows that long are tiled 64 cells by 8 rows.
+inline int check_tiles3(const rsg_grid *g) {
+    if (!tiles_fit(g->nx, g->ny, R3 * B3 / 64, std::min(std::max(g->order, 1), 8)))
+        return fail(RSG_EINVAL, "e3d: rows too long for 32-bit offsets (nx min(ny, 8 + 2 order) >= 2^30)");
+    return RSG_OK;
+}
 inline G3 make_g3e(const rsg_grid *g, const rsg_state_e3d *s) {
     return make_g3(g, s->tab, std::min(std::max(g->order, 1), 8));
 }

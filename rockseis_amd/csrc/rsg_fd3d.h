@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "rsg_common.h"
+#include "rsg_tiles3.h"
 
 namespace rsg {
 
@@ -53,13 +54,9 @@ constexpr int R3 = 2, B3 = 256;  // rows a thread, threads a block
 // 222 us on 320 x 300 x 280 at order 8 where four take 248 + 185; five spill.
 #define RSG3_BOUNDS __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu(4, 8)))
 
-// Raw buffers over the tile's part of an array: every lane either has an
-// offset inside its tile's window of the grid, or kOut, which no descriptor
-// covers: loads return 0 and stores are dropped, so lanes outside the grid
-// need no branches.  A descriptor that is not live covers nothing.
-constexpr unsigned kOut = 0xFFFFFF00u;
+// The tile's part of an array; a descriptor that is not live covers nothing.
 __device__ __forceinline__ Buf tile_buf(const float *f, long off, bool live = true) {
-    return mkbuf(f + off, live ? 0x7FFFFF00u : 0u);
+    return mkbuf(f + off, live ? kOut : 0u);
 }
 
 // A uniform value the optimiser may not see through (v is uniform;
@@ -208,23 +205,27 @@ __device__ __forceinline__ float dfw_edge(const float *s, int st, int k, float i
 }
 
 // Window of one plane, TY + 2*HY rows of TX + 2*HX: each thread's element
-// list (offsets from the window's corner, kOut outside the grid) is fixed for
-// the whole march; fetch loads into registers, store writes them to LDS.
+// list (offsets from the corner of the window's rows inside the grid, kOut
+// outside it) is fixed for the whole march; fetch loads into registers, store
+// writes them to LDS.
 template <int TX, int HX, int HY>
 struct Win3 {
     static constexpr int LD = TX + 2 * HX, N = LD * (R3 * B3 / TX + 2 * HY), K = (N + B3 - 1) / B3;
     unsigned off[K];
+    long corner;  // from the tile's first cell to the base of the offsets
     __device__ __forceinline__ void init(int nx, int ny, int x0, int y0) {
+        const int row0 = HY ? window_row0(y0, HY) : y0;
+        corner = HY ? (long)(row0 - y0) * nx - HX : -HX;
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int i = (int)threadIdx.x + k * B3, r = i / LD, c = i - r * LD;
             const int y = y0 - HY + r, x = x0 - HX + c;
-            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? (unsigned)((r * nx + c) * 4) : kOut;
+            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? tile_off(y - row0, nx, c) : kOut;
         }
     }
     // f at plane offset `at` (of the tile's first cell)
-    __device__ __forceinline__ void fetch(float (&v)[K], const float *f, long at, int nx, bool live) const {
-        const Buf b = tile_buf(f, at - (long)HY * nx - HX, live);
+    __device__ __forceinline__ void fetch(float (&v)[K], const float *f, long at, bool live) const {
+        const Buf b = tile_buf(f, at + corner, live);
 #pragma unroll
         for (int k = 0; k < K; k++) v[k] = b.ld(off[k], 0);
     }
@@ -272,7 +273,7 @@ struct Lane3 {
 #pragma unroll
         for (int r = 0; r < R3; r++) {
             ok[r] = x < g.nx && y + r < g.ny;
-            oc[r] = ok[r] ? (unsigned)(((ty * R3 + r) * g.nx + tx) * 4) : kOut;
+            oc[r] = ok[r] ? tile_off(ty * R3 + r, g.nx, tx) : kOut;
         }
         t0 = (long)p.y0 * g.nx + p.x0;
     }
@@ -469,8 +470,8 @@ struct Div3 {
         auto window = [&](int z, int k) RSG_INLINE {
             const bool live = z < ze;
             const long at = opaque(o + k * nxy);
-            if (HX) wx.fetch(wvx, f[0], at, nx, live);
-            if (HY) wy.fetch(wvy, f[1], at, nx, live);
+            if (HX) wx.fetch(wvx, f[0], at, live);
+            if (HY) wy.fetch(wvy, f[1], at, live);
         };
         auto own = [&](int z, int k) RSG_INLINE {
             const bool live = z < ze;
@@ -634,7 +635,7 @@ struct Grad3 {
         float V[3][R3], R[3][R3], sx[R3], sy[R3], wv[W::K], q[R3][2 * H + 2], qn[2][R3];
         ZVals zv;
         auto window = [&](int z, int k) RSG_INLINE {
-            w.fetch(wv, P, opaque(o + k * nxy), nx, z < ze);
+            w.fetch(wv, P, opaque(o + k * nxy), z < ze);
         };
         auto own = [&](int z, int k) RSG_INLINE {
             const bool live = z < ze;
