@@ -44,8 +44,6 @@
 
 namespace rsg {
 
-constexpr int R3 = 2, B3 = 256;  // rows a thread, threads a block
-
 // Lambdas of the march: one left out of line would put the arrays it captures,
 // the queue among them, in scratch memory.
 #define RSG_INLINE __attribute__((always_inline))
@@ -76,69 +74,10 @@ struct Term3 {
     int fw;
 };
 
-// Tile order.  ncx x ncy columns of TX x TY cells; the z planes in three
-// zones (strips or shortened stencils at the low face, neither, the high
-// face), zone i of planes z[i] .. z[i+1]-1 in n[i] chunks of zc planes; ncomp
-// components (blocks that update different arrays of one tile from partly the
-// same inputs), the first `first` (0 or 1) of them before all others.  With xgroups blocks are dealt round-robin to the 8 XCDs (XCD
-// k runs blocks k, k+8, ...) and XCD k marches its own contiguous group of
-// columns cg[k] .. cg[k+1]-1 through the chunks, components fastest (those
-// after the first), then columns: the blocks an XCD holds at once are neighbours at the same depth,
-// so shared inputs, halos and the lines that tile rows share are fetched into
-// that XCD's L2 once.
-struct Tiles3 {
-    int tx, xgroups, ncx, ncy, zc, ncomp, first;
-    int z[4], n[3];
-    int cg[9];
-};
-
-struct Pos3 {
-    int x0, y0, zb, ze, comp, zone;
-};
-
-// Component of block r of n blocks a component; r: its block.
-__device__ __forceinline__ bool comp_of(const Tiles3 &t, int n, int &r, int &comp) {
-    const int m = t.ncomp - t.first;
-    comp = 0;
-    if (r >= t.first * n) {
-        r -= t.first * n;
-        comp = t.first + r % m;
-        r /= m;
-    }
-    return r < n;
-}
-
+// Tile, chunk and component of this block; false for surplus blocks.
 template <int TX>
 __device__ __forceinline__ bool tile3_of(const Tiles3 &t, Pos3 &p) {
-    int col, ck, r = blockIdx.x;
-    const int nck = t.n[0] + t.n[1] + t.n[2];
-    if (!t.xgroups) {
-        if (!comp_of(t, t.ncx * t.ncy * nck, r, p.comp)) return false;
-        ck = r / (t.ncx * t.ncy);
-        col = r - ck * (t.ncx * t.ncy);
-    } else {
-        const int k = r % 8, ncol = t.cg[k + 1] - t.cg[k];
-        r /= 8;
-        if (ncol <= 0 || !comp_of(t, ncol * nck, r, p.comp)) return false;
-        ck = r / ncol;
-        col = t.cg[k] + (r - ck * ncol);
-    }
-    const int cy = col / t.ncx;
-    p.x0 = (col - cy * t.ncx) * TX;
-    p.y0 = cy * (R3 * B3 / TX);
-    int zone = 0;
-    if (ck >= t.n[0]) {
-        ck -= t.n[0];
-        zone = 1;
-        if (ck >= t.n[1]) {
-            ck -= t.n[1];
-            zone = 2;
-        }
-    }
-    p.zb = t.z[zone] + ck * t.zc;
-    p.ze = min(p.zb + t.zc, t.z[zone + 1]);
-    p.zone = zone;
-    return p.zb < p.ze;
+    return tile3_at<TX>(t, blockIdx.x, p);
 }
 
 // Grid, step and stencil description every 3D kernel takes.
@@ -151,12 +90,9 @@ struct G3 {
     Tiles3 t;
 };
 
-// Does the tile hold cells of x or y strips, or whose x or y stencils the
-// array's ends shorten, or cells outside the grid?
 template <int TX>
 __device__ __forceinline__ bool tile_pxy(const G3 &g, const Pos3 &p) {
-    const int m = max(g.lpml, g.order);
-    return p.x0 < m || p.x0 + TX > g.nx - m || p.y0 < m || p.y0 + R3 * B3 / TX > g.ny - m;
+    return tile_pxy(TX, g.nx, g.ny, g.lpml, g.order, p);
 }
 
 // z-derivative from a queue q[j] = f(z + off + j): both the forward
@@ -755,49 +691,7 @@ static G3 make_g3(const rsg_grid *g, const float *tab, int order) {
 
 // Launch grid of ncomp components, and the tile order.
 static unsigned layout3(G3 &k, int ncomp, int first = 0) {
-    Tiles3 &t = k.t;
-    // Rows of 64 touch fewer partly used cache lines (440^3, order 4: 778 + 474
-    // us a step against 873 + 514 with 32), unless they waste much more of a
-    // narrow grid's last tile (160 x 150 x 140: 36 + 33 us against 33 + 29).
-    const int w64 = (k.nx + 63) / 64 * 64, w32 = (k.nx + 31) / 32 * 32;
-    t.tx = 10 * w64 <= 11 * w32 ? 64 : 32;
-    const int ty = R3 * B3 / t.tx;
-    t.ncx = (k.nx + t.tx - 1) / t.tx;
-    t.ncy = (k.ny + ty - 1) / ty;
-    t.ncomp = ncomp;
-    t.first = first;
-    // the low zone ends before the high strip, so that a chunk has one face
-    const int m = std::max(k.lpml, k.order), lo = std::min(m, k.nz - k.lpml), hi = std::max(lo, k.nz - m);
-    t.z[0] = 0;
-    t.z[1] = lo;
-    t.z[2] = hi;
-    t.z[3] = k.nz;
-    const long cols = (long)t.ncx * t.ncy * ncomp;
-    auto split = [&](int zc) {
-        t.zc = zc;
-        for (int i = 0; i < 3; i++) t.n[i] = (t.z[i + 1] - t.z[i] + zc - 1) / zc;
-        return t.n[0] + t.n[1] + t.n[2];
-    };
-    int zc = tuning().zc3d;
-    if (zc <= 0) {
-        // Short chunks give many blocks, long ones amortise the queue's
-        // filling: 8 planes where that gives enough blocks, else 4.  One
-        // component: four rounds (320 x 300 x 280: 229 + 154 us a step with 8,
-        // 230 + 161 with 4; 200 x 190 x 180, 2400 blocks: 69 + 50 with 8, 62 +
-        // 50 with 4).  The elastic components' blocks do less each and start
-        // cheaper on lines their neighbours read: two rounds (140 x 130 x 120:
-        // 50 + 60 us with 8, 53 + 64 with 4; 70 x 60 x 50: 21 + 23, 16 + 16).
-        zc = cols * split(8) >= (ncomp > 1 ? 2048 : 4096) ? 8 : 4;
-    }
-    const int nck = split(zc), ncol = t.ncx * t.ncy;
-    t.xgroups = tuning().xcd3d ? 1 : 0;
-    if (!t.xgroups) return (unsigned)((long)ncol * nck * ncomp);
-    int most = 0;
-    for (int x = 0; x <= 8; x++) {
-        t.cg[x] = (int)((long)ncol * x / 8);
-        if (x) most = std::max(most, t.cg[x] - t.cg[x - 1]);
-    }
-    return (unsigned)(8L * most * nck * ncomp);
+    return layout_tiles3(k.t, k.nx, k.ny, k.nz, k.lpml, k.order, ncomp, first, tuning().zc3d, tuning().xcd3d);
 }
 
 #define RSG3_ORDER_CASES(LAUNCH, X, ORDER) \

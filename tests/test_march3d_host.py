@@ -14,11 +14,51 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 KOUT = 0xFFFFFF00  # no descriptor covers offsets from here on
 
 HARNESS = r"""
+#include <vector>
+
 #include "rsg_tiles3.h"
 extern "C" {
 unsigned off(int r, int nx, int c) { return rsg::tile_off(r, nx, c); }
 int row0(int y0, int hy) { return rsg::window_row0(y0, hy); }
 int fit(int nx, int ny, int ty, int order) { return rsg::tiles_fit(nx, ny, ty, order); }
+
+// The layout of a launch of ncomp components: out = {blocks, tx, zc, xgroups}.
+void layout(const int *a, unsigned *out) {
+    rsg::Tiles3 t;
+    out[0] = rsg::layout_tiles3(t, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8]);
+    out[1] = t.tx;
+    out[2] = t.zc;
+    out[3] = t.xgroups;
+}
+
+// Walks all blocks.  0: every plane of every tile is marched once a component,
+// by a chunk that holds planes of one face's strip and shortened stencils or,
+// in the middle zone, of none; else what is wrong.  kinds: bit 2 pxy + pz set
+// where a block takes that instantiation.
+int cover(const int *a, int *kinds) {
+    const int nx = a[0], ny = a[1], nz = a[2], lpml = a[3], order = a[4], ncomp = a[5];
+    rsg::Tiles3 t;
+    const unsigned n = rsg::layout_tiles3(t, nx, ny, nz, lpml, order, ncomp, a[6], a[7], a[8]);
+    const int ty = rsg::R3 * rsg::B3 / t.tx, m = std::max(lpml, order);
+    std::vector<int> seen((size_t)t.ncx * t.ncy * nz * ncomp);
+    *kinds = 0;
+    for (unsigned r = 0; r < n; r++) {
+        rsg::Pos3 p{};
+        if (!(t.tx == 64 ? rsg::tile3_at<64>(t, (int)r, p) : rsg::tile3_at<32>(t, (int)r, p))) continue;
+        if (p.x0 % t.tx || p.y0 % ty || p.x0 >= nx || p.y0 >= ny || p.comp < 0 || p.comp >= ncomp) return 1;
+        if (p.zb < 0 || p.ze > nz || p.ze - p.zb > t.zc) return 2;
+        for (int z = p.zb; z < p.ze; z++) {
+            seen[(((size_t)z * t.ncy + p.y0 / ty) * t.ncx + p.x0 / t.tx) * ncomp + p.comp]++;
+            if (p.zone == 1 && (z < m || z >= nz - m)) return 3;
+            if (p.zone == 0 && z >= nz - lpml) return 4;
+            if (p.zone == 2 && z < lpml) return 5;
+        }
+        *kinds |= 1 << (2 * rsg::tile_pxy(t.tx, nx, ny, lpml, order, p) + (p.zone != 1));
+    }
+    for (int s : seen)
+        if (s != 1) return 6;
+    return 0;
+}
 }
 """
 
@@ -33,6 +73,34 @@ def march(tmp_path_factory):
     lib = C.CDLL(str(so))
     lib.off.restype = C.c_uint
     return lib
+
+
+def _layout(m, *args):
+    out = (C.c_uint * 4)()
+    m.layout((C.c_int * 9)(*args), out)
+    return dict(zip(("blocks", "tx", "zc", "xgroups"), out))
+
+
+def test_every_plane_of_every_tile_is_marched_once(march):
+    rng = random.Random(3)
+    for i in range(400):
+        order, lpml = rng.randint(1, 8), rng.randint(1, 20)
+        n = [max(2 * lpml + 1, int(10 ** rng.uniform(0.5, 2.5))) for _ in range(3)]
+        ncomp, first = rng.choice(((1, 0), (3, 0), (4, 1)))
+        zc, xcd = rng.choice((0, 0, 1, 2, 3, 8, 16, 4096)), rng.randint(0, 1)
+        a = (C.c_int * 9)(*n, lpml, order, ncomp, first, zc, xcd)
+        kinds = C.c_int()
+        assert march.cover(a, C.byref(kinds)) == 0, list(a)
+
+
+# padded nx, ny, nz, components, zc3d: thin grids, and very large ones with
+# short chunks asked for, whose blocks of 256 threads passed 2^32 threads
+@pytest.mark.parametrize("nx,ny,nz,ncomp,zc", [(3, 8192, 65535, 4, 0), (3, 12000, 65535, 3, 0),
+                                               (1300, 1300, 1300, 4, 1), (1400, 1400, 1400, 3, 1)])
+def test_a_launch_holds_its_blocks(march, nx, ny, nz, ncomp, zc):
+    for xcd in (0, 1):
+        t = _layout(march, nx, ny, nz, 1, 8, ncomp, ncomp // 4, zc, xcd)
+        assert 0 < t["blocks"] * 256 < 1 << 32, t
 
 
 def _window_offsets(m, nx, ny, ty, order):
