@@ -19,11 +19,12 @@ constexpr int R3 = 2, B3 = 256;  // rows a thread, threads a block
 // components (blocks that update different arrays of one tile from partly the
 // same inputs), the first `first` (0 or 1) of them before all others.  With
 // xgroups blocks are dealt round-robin to the 8 XCDs (XCD k runs blocks k,
-// k+8, ...) and XCD k marches its own contiguous group of columns
+// k+8, ...).  xgroups 1: XCD k marches its own contiguous group of columns
 // cg[k] .. cg[k+1]-1 through the chunks, components fastest (those after the
 // first), then columns: the blocks an XCD holds at once are neighbours at the
 // same depth, so shared inputs, halos and the lines that tile rows share are
-// fetched into that XCD's L2 once.
+// fetched into that XCD's L2 once.  xgroups 2, for few columns: XCD k marches
+// an eighth of all chunks, those of one depth after those of the one before.
 struct Tiles3 {
     int tx, xgroups, ncx, ncy, zc, ncomp, first;
     int z[4], n[3];
@@ -55,6 +56,12 @@ RSG_HD bool tile3_at(const Tiles3 &t, int r, Pos3 &p) {
         if (!comp_of(t, t.ncx * t.ncy * nck, r, p.comp)) return false;
         ck = r / (t.ncx * t.ncy);
         col = r - ck * (t.ncx * t.ncy);
+    } else if (t.xgroups == 2) {
+        const int k = r % 8, ncol = t.ncx * t.ncy, i0 = (int)((long)ncol * nck * k / 8);
+        r /= 8;
+        if (!comp_of(t, (int)((long)ncol * nck * (k + 1) / 8) - i0, r, p.comp)) return false;
+        ck = (i0 + r) / ncol;
+        col = i0 + r - ck * ncol;
     } else {
         const int k = r % 8, ncol = t.cg[k + 1] - t.cg[k];
         r /= 8;
@@ -122,19 +129,33 @@ inline unsigned layout_tiles3(Tiles3 &t, int nx, int ny, int nz, int lpml, int o
     // rounds (320 x 300 x 280: 229 + 154 us a step with 8, 230 + 161 with 4;
     // 200 x 190 x 180, 2400 blocks: 69 + 50 with 8, 62 + 50 with 4).  The
     // elastic components' blocks do less each and start cheaper on lines their
-    // neighbours read: two rounds (140 x 130 x 120: 50 + 60 us with 8, 53 + 64
-    // with 4; 70 x 60 x 50: 21 + 23, 16 + 16).
-    if (zc <= 0) zc = ncol * ncomp * split(8) >= (ncomp > 1 ? 2048 : 4096) ? 8 : 4;
-    t.xgroups = xcd ? 1 : 0;
+    // neighbours read: one and a half (140 x 130 x 120: 50 + 60 us with 8, 53 +
+    // 64 with 4; 33 x 500 x 33: 26 + 28, 26 + 31; 120 x 110 x 100, velocity, 1092
+    // blocks: 36, 32).  Where all their blocks run at once a step lasts as long
+    // as one block, and chunks of 1 or 2 planes end sooner: three or four
+    // blocks a compute unit (order 4: 24^3 12 + 13 us with 4 planes, 6.2 + 6.6
+    // with 1; 64^3 13.7 + 13.9 with 4, 11.1 + 11.8 with 2, 13.6 + 15.7 with 1).
+    if (zc <= 0) {
+        zc = ncol * ncomp * split(8) >= (ncomp > 1 ? 1536 : 4096) ? 8 : 4;
+        for (int c = 2; c >= 1 && ncomp > 1; c--)
+            if (ncol * ncomp * split(c) <= (c == 2 ? 1024 : 768)) zc = c;
+    }
     long most = 0;  // columns of the largest group
     for (int x = 0; x <= 8; x++) {
         t.cg[x] = (int)(ncol * x / 8);
         if (x) most = std::max(most, (long)t.cg[x] - t.cg[x - 1]);
     }
+    // Few columns split unevenly: where the largest group is more than an
+    // eighth above the mean, elastic launches are split by depth (order 4, us a
+    // velocity + a stress step by columns, by depth: 20 x 20 x 400, 2 columns, 6 of
+    // 8 XCDs idle: 34 + 41, 15 + 16; 60 x 40 x 1000: 71 + 86, 44 + 63; 120 x 110 x
+    // 100, 28 columns: 35 + 41, 33 + 37; 90 x 64 x 64: 15.6 + 19.1, 16.1 + 15.6).
+    t.xgroups = !xcd ? 0 : (ncomp == 1 || 64 * most <= 9 * ncol ? 1 : 2);
     // Longer chunks where these give more blocks than a launch holds (thin or
     // very large grids, a small zc3d)
     for (zc = std::min(zc, nz);; zc = std::min(2 * zc, nz)) {
-        const long blocks = (t.xgroups ? 8 * most : ncol) * split(zc) * ncomp;
+        const long nck = split(zc);
+        const long blocks = (t.xgroups == 2 ? (ncol * nck + 7) / 8 * 8 : (t.xgroups ? 8 * most : ncol) * nck) * ncomp;
         if (blocks <= kMaxBlocks || zc == nz) return (unsigned)blocks;
     }
 }

@@ -31,6 +31,20 @@ void layout(const int *a, unsigned *out) {
     out[3] = t.xgroups;
 }
 
+// The most blocks one XCD (r mod 8) holds, in percent of an eighth of all.
+int share(const int *a) {
+    rsg::Tiles3 t;
+    const unsigned n = rsg::layout_tiles3(t, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8]);
+    long live[8] = {}, all = 0;
+    for (unsigned r = 0; r < n; r++) {
+        rsg::Pos3 p{};
+        const int l = t.tx == 64 ? rsg::tile3_at<64>(t, (int)r, p) : rsg::tile3_at<32>(t, (int)r, p);
+        live[r % 8] += l;
+        all += l;
+    }
+    return (int)(*std::max_element(live, live + 8) * 800 / all);
+}
+
 // Walks all blocks.  0: every plane of every tile is marched once a component,
 // by a chunk that holds planes of one face's strip and shortened stencils or,
 // in the middle zone, of none; else what is wrong.  kinds: bit 2 pxy + pz set
@@ -91,6 +105,22 @@ def test_every_plane_of_every_tile_is_marched_once(march):
         a = (C.c_int * 9)(*n, lpml, order, ncomp, first, zc, xcd)
         kinds = C.c_int()
         assert march.cover(a, C.byref(kinds)) == 0, list(a)
+
+
+# padded nx, ny, nz, lpml of small and of thin grids, and of one that fills the chip
+@pytest.mark.parametrize("grid", [(24, 24, 24, 4), (32, 32, 32, 6), (48, 48, 48, 10), (64, 64, 64, 10), (70, 60, 50, 10),
+                                  (20, 20, 400, 4), (400, 20, 20, 4), (20, 400, 20, 4), (33, 500, 33, 10),
+                                  (140, 130, 120, 20)], ids=str)
+def test_elastic_launches_spread_over_the_chip(march, grid):
+    """No XCD gets more than an eighth above its share of the blocks, and a
+    grid whose blocks all run at once is cut in chunks of one or two planes."""
+    nx, ny, nz, lpml = grid
+    for ncomp in (3, 4):
+        a = (nx, ny, nz, lpml, 4, ncomp, ncomp // 4, 0, 1)
+        assert march.share((C.c_int * 9)(*a)) <= 113, a
+        t = _layout(march, *a)
+        cols = -(-nx // t["tx"]) * -(-ny // (512 // t["tx"]))
+        assert t["zc"] <= 2 or cols * ncomp * nz // 2 > 1000, t
 
 
 # padded nx, ny, nz, components, zc3d: thin grids, and very large ones with
