@@ -617,10 +617,18 @@ __device__ __forceinline__ void e2d_velocity_body(const K2D &a, int x0, int z0, 
     StripX<RZ, FAST> pxx, pxz;    // of Sxx and Sxz
     StripZ<RZ, FAST> pzxz, pzz;   // of Sxz and Szz
 #define PSI_(S, LO, HI) a.psi[RSG_E2D_##S##_##LO], a.psi[RSG_E2D_##S##_##HI], a.psi[RSG_E2D_##S##_##LO], a.psi[RSG_E2D_##S##_##HI]
-    pxx.load(pl, tb, 1, PSI_(SXX, LEFT, RIGHT), xo);
-    pxz.load(pl, tb, 0, PSI_(SXZX, LEFT, RIGHT), xo);
-    pzxz.load(pl, tb, 0, PSI_(SXZZ, TOP, BOTTOM), zo, x);
-    pzz.load(pl, tb, 1, PSI_(SZZ, TOP, BOTTOM), zo, x);
+    // Adjoint state: the window loads hold up to four registers a value (Ld4),
+    // and with the strips' in flight beside them RZ = 2 needs 102 VGPRs at order
+    // 8, four waves a SIMD; after the windows are in LDS, 72 and seven.  Interior
+    // tiles pay for boundary ones there (us, together -> after: 5000 x 4000 order
+    // 8 320 -> 290, 32 shots of 861 x 461 193 -> 163, RZ = 8 613 -> 370).
+    auto strips = [&]() __attribute__((always_inline)) {
+        pxx.load(pl, tb, 1, PSI_(SXX, LEFT, RIGHT), xo);
+        pxz.load(pl, tb, 0, PSI_(SXZX, LEFT, RIGHT), xo);
+        pzxz.load(pl, tb, 0, PSI_(SXZZ, TOP, BOTTOM), zo, x);
+        pzz.load(pl, tb, 1, PSI_(SZZ, TOP, BOTTOM), zo, x);
+    };
+    if (!BW) strips();
     const float cev = edge_fetch<FAST>();
     Tile<TZ, H, 0> txx;
     Tile<TZ, 0, H> tzz;
@@ -640,6 +648,7 @@ __device__ __forceinline__ void e2d_velocity_body(const K2D &a, int x0, int z0, 
     tile_store(txx, sXX);
     tile_store(tzz, sZZ);
     tile_store(txz, sXZ);
+    if (BW) strips();
     __syncthreads();
     if (!xin) return;
     const int kxf = FAST ? ORDER : kfw(x, nx, ORDER), kxb = FAST ? ORDER : kbw(x, nx, ORDER);
