@@ -311,7 +311,11 @@ def cpu_configs(n_window):
     (numforw(nt, 50) + nt) steps of the Revolve schedule (the imaging
     condition and checkpoint copies not counted).  Config 4's 440^3 grid
     takes about a minute per reference step on one core and is left out of
-    the default run."""
+    the default run.  Where the reference build is absent nothing is timed:
+    the oracle's restatement starts no run in its middle."""
+    import oracle
+    if not oracle.ref_available():
+        return {"skipped": "reference build absent (make -C oracle ref, where the reference's sources are mounted)"}
     import numpy as np
     import torch
     from oracle import runs
