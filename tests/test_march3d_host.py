@@ -107,6 +107,20 @@ def test_every_plane_of_every_tile_is_marched_once(march):
         assert march.cover(a, C.byref(kinds)) == 0, list(a)
 
 
+def test_the_half_step_tests_reach_every_march(march):
+    """The sizes the march is compared with the oracle at hold tiles and chunks
+    with and without strips or shortened stencils, in both tile widths."""
+    from tests.test_gpu_march3d import INNER, SIZES
+    for ncomp in (1, 3, 4):
+        kinds = {32: 0, 64: 0}
+        for size in SIZES + INNER:
+            a = (C.c_int * 9)(*size, ncomp, ncomp // 4, 0, 1)
+            k = C.c_int()
+            assert march.cover(a, C.byref(k)) == 0
+            kinds[_layout(march, *a)["tx"]] |= k.value
+        assert kinds == {32: 15, 64: 15}
+
+
 # padded nx, ny, nz, lpml of small and of thin grids, and of one that fills the chip
 @pytest.mark.parametrize("grid", [(24, 24, 24, 4), (32, 32, 32, 6), (48, 48, 48, 10), (64, 64, 64, 10), (70, 60, 50, 10),
                                   (20, 20, 400, 4), (400, 20, 20, 4), (20, 400, 20, 4), (33, 500, 33, 10),
