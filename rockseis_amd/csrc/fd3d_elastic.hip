@@ -31,7 +31,7 @@ namespace rsg {
 namespace {
 
 struct K3E {
-    int nx, ny, nz, lpml, fs, order;
+    int nx, ny, nz, lpml, order;
     float dt, invd[3];
     const float *tab;
     float *V[3], *Sxx, *Syy, *Szz, *Syz, *Sxz, *Sxy;
@@ -283,7 +283,6 @@ K3E make_k3e(const rsg_grid *g, const rsg_state_e3d *s) {
     k.ny = g->ny;
     k.nz = g->nz;
     k.lpml = g->lpml;
-    k.fs = g->fs;
     k.order = g->order < 1 ? 1 : (g->order > 8 ? 8 : g->order);
     k.dt = g->dt;
     const float d[3] = {g->dx, g->dy, g->dz};

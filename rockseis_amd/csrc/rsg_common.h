@@ -123,15 +123,6 @@ __device__ __forceinline__ float dbw_k(const float *s, int st, int k, float invd
     return acc * invd;
 }
 
-// CFS-PML memory update and field correction (waves.cpp:258-263 pattern):
-// psi = B*psi + A*d; F -= dt*M*(psi + C*d)
-__device__ __forceinline__ void pml_corr(float &F, float dtM, float *psi, float A, float B, float C,
-                                         float d) {
-    float p = B * (*psi) + A * d;
-    *psi = p;
-    F -= dtM * (p + C * d);
-}
-
 // PML table rows (pml.h:60-74)
 enum { T_A = 0, T_B = 1, T_C = 2, T_STAG = 3, T_RBB = 6 };
 

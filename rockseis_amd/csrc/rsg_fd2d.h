@@ -200,8 +200,6 @@ struct Tile {
     float a[KR], b[KR];
 };
 
-__device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
-
 template <int TZ, int HX, int HZ, bool FAST, class F>
 __device__ __forceinline__ void tile_fetch(Tile<TZ, HX, HZ> &t, F &&ld, int nx, int nz, int x0, int z0) {
     using T = Tile<TZ, HX, HZ>;
