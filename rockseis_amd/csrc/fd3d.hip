@@ -6,7 +6,10 @@
 namespace rsg {
 
 // The queue, three fields and three moduli are a few registers too many for
-// four waves a SIMD from order 7 on (four spill 16 bytes a lane).
+// four waves a SIMD from order 7 on (four spill 20 and 60 bytes a lane).  us at
+// order 8, three waves against four with their spills: 120 x 110 x 100 22.9, 25.0,
+// 140 x 130 x 120 36.3, 38.2, 160 x 150 x 140 46.0, 41.8, 200 x 190 x 180 76.8, 70.0,
+// 320 x 300 x 280 251, 250, 440^3 822, 822.
 template <int TX, int ORDER>
 __global__ __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu((ORDER) >= 7 ? 3 : 4, 8))) void a3d_velocity_kernel(const G3 g, const Grad3Args a) {
     using K = Grad3<TX, ORDER>;

@@ -146,11 +146,13 @@ inline unsigned layout_tiles3(Tiles3 &t, int nx, int ny, int nz, int lpml, int o
         if (x) most = std::max(most, (long)t.cg[x] - t.cg[x - 1]);
     }
     // Few columns split unevenly: where the largest group is more than an
-    // eighth above the mean, elastic launches are split by depth (order 4, us a
-    // velocity + a stress step by columns, by depth: 20 x 20 x 400, 2 columns, 6 of
-    // 8 XCDs idle: 34 + 41, 15 + 16; 60 x 40 x 1000: 71 + 86, 44 + 63; 120 x 110 x
-    // 100, 28 columns: 35 + 41, 33 + 37; 90 x 64 x 64: 15.6 + 19.1, 16.1 + 15.6).
-    t.xgroups = !xcd ? 0 : (ncomp == 1 || 64 * most <= 9 * ncol ? 1 : 2);
+    // eighth above the mean, the chunks are split by depth (us a velocity + a
+    // stress step by columns, by depth; elastic, order 4: 20 x 20 x 400, 2 columns,
+    // 6 of 8 XCDs idle: 34 + 41, 15 + 16; 60 x 40 x 1000: 71 + 86, 44 + 63; 120 x
+    // 110 x 100, 28 columns: 35 + 41, 33 + 37; 90 x 64 x 64: 15.6 + 19.1, 16.1 +
+    // 15.6; acoustic: 120 x 110 x 100 order 4 18.6 + 17.3, 16.6 + 16.0, order 8,
+    // where three blocks a compute unit are resident, 31.2 + 25.1, 22.9 + 23.0).
+    t.xgroups = !xcd ? 0 : (64 * most <= 9 * ncol ? 1 : 2);
     // Longer chunks where these give more blocks than a launch holds (thin or
     // very large grids, a small zc3d)
     for (zc = std::min(zc, nz);; zc = std::min(2 * zc, nz)) {
