@@ -133,11 +133,11 @@ int rsg_zero(void *ptr, size_t bytes, void *stream);
  * in percent of a PML / edge cell or tile against an interior one when the 2D
  * tiles are split into eight XCD ranges of equal cost, default 200), "zc3d"
  * (z planes per 3D block, 0 = automatic), "xcd3d" (3D tile order: 1 = each XCD
- * marches its own contiguous group of (x, y) columns through z, 0 = grid
- * order; default 1), "fuse_io" (modelling runs: sources and velocity gathers
- * in the stress kernel, 1 = on).  Results do not depend
- * on them; rockseis_amd.autotune picks rz2d, pml_cost and zc3d per
- * workload. */
+ * marches its own contiguous group of (x, y) columns through z or, where the
+ * columns split unevenly, its own eighth of the depths; 0 = grid order;
+ * default 1), "fuse_io" (modelling runs: sources and velocity gathers in the
+ * stress kernel, 1 = on).  Results do not depend on them;
+ * rockseis_amd.autotune picks rz2d, pml_cost and zc3d per workload. */
 int rsg_set_tuning(const char *key, int value);
 int rsg_get_tuning(const char *key, int *value);
 

@@ -4,12 +4,12 @@ The fused 2D kernels give each thread ``rz2d`` rows of a 64-wide tile
 (1, 2, 4 or 8) and split the tiles into eight contiguous XCD ranges of equal
 estimated cost, a PML / edge tile counting ``pml_cost`` percent of an
 interior one; the 3D kernels march ``zc3d`` z planes per block (0 = chosen
-from the grid so that a launch has >= 2048 blocks).  Results do not depend on
-any knob (every cell is computed by the same arithmetic), only the time
-does, so the tuner times a velocity + stress half-step pair for every
-candidate on a zeroed scratch state of the caller's shape, keeps the fastest
-and sets it with ``rsg_set_tuning`` (2D: rz2d first, then pml_cost at that
-rz2d).  Choices are cached per
+from the grid: acoustic, 8 where that gives at least 4096 blocks, else 4).
+Results do not depend on any knob (every cell is computed by the same
+arithmetic), only the time does, so the tuner times a velocity + stress
+half-step pair for every candidate on a zeroed scratch state of the caller's
+shape, keeps the fastest and sets it with ``rsg_set_tuning`` (2D: rz2d first,
+then pml_cost at that rz2d).  Choices are cached per
 (kind, padded grid, order, shots) in-process and, if ``RSG_TUNE_CACHE`` names
 a JSON file, across processes.
 """

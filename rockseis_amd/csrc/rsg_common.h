@@ -130,10 +130,10 @@ enum { T_A = 0, T_B = 1, T_C = 2, T_STAG = 3, T_RBB = 6 };
 struct Tuning {
     int rz2d = 2;   // rows per thread of the 2D tiles: 1, 2, 4 or 8
     int rz2d_ragged = 2;  // the same for the ragged batches (elastic FWI windows)
-    int zc3d = 0;   // z planes per 3D block (0: automatic)
+    int zc3d = 0;   // z planes per 3D block (0: automatic; longer where a launch cannot hold the blocks)
     int fuse_io = 1;  // modelling runs: source injection / velocity gathers in the stress kernel
     int pml_cost = 200;  // weight (percent of an interior tile) of a PML / edge tile in the XCD split
-    int xcd3d = 1;  // 3D tiles: 1 = each XCD marches its own contiguous group of (x, y) columns, 0 = grid order
+    int xcd3d = 1;  // 3D tiles: 1 = each XCD marches its own group of (x, y) columns or, where these split unevenly, of depths, 0 = grid order
 };
 Tuning &tuning();
 

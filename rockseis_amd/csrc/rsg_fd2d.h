@@ -191,9 +191,9 @@ __host__ __device__ inline bool interior_tile(const K2D &a, int x0, int z0, int 
 // every global load of a block is in flight before the first LDS write: fetch
 // issues all loads into registers (thread row ty takes window rows ty, ty+4,
 // ...; columns tx and, for halo columns, tx+64), store writes them out.
-// Boundary tiles clamp the address into the grid and select 0 outside it, so
-// the loads stay unconditional; zeros outside the grid are never read by the
-// reduced edge stencils.
+// Boundary tiles load without branches too: rows outside the grid lie outside
+// the buffer (0), columns outside it are replaced by 0 after the load; the
+// reduced edge stencils read none of them.
 template <int TZ, int HX, int HZ>
 struct Tile {
     static constexpr int LD = BX + 2 * HX, ROWS = TZ + 2 * HZ, KR = (ROWS + BZ - 1) / BZ;

@@ -19,22 +19,25 @@
 // of a chunk use an empty descriptor.  Two planes ahead (a second set of
 // registers) costs order 8 its fourth wave a SIMD, which hides more.
 //
-// What bounds it: HBM on large grids, the march's latency and the filling of
-// the queue on small ones.  Against the kernels before (acoustic: 64 x 8 tiles
-// that loaded the memory variables where they were used; elastic: a thread a
-// cell, all taps through L1 and L2), us a velocity + a stress half step:
-//   acoustic, order 4:  320 x 300 x 280  333 + 256 -> 235 + 163 (4.6, 4.0 TB/s
-//                       of its arrays once), 440^3  914 + 677 -> 769 + 467,
-//                       160 x 150 x 140  66 + 58 -> 32 + 29,
-//                       120 x 110 x 100  42 + 36 -> 19 + 18
-//   acoustic, order 8:  320 x 300 x 280  519 + 445 -> 248 + 185
-//   elastic, order 4:   200 x 190 x 180  286 + 316 -> 143 + 188,
-//                       140 x 130 x 120  80 + 85 -> 50 + 61,
-//                       70 x 60 x 50  17.2 + 17.2 -> 15.7 + 15.9
-//   elastic, order 8:   200 x 190 x 180  415 + 447 -> 177 + 218,
-//                       240^3  671 + 731 -> 287 + 371
-// The elastic steps reach 2.2 to 2.9 TB/s of their arrays once: three or four
-// blocks read each field's window and queue, from L2 for the most part.
+// What bounds it: HBM on large acoustic grids (440^3, order 4: velocity 4.25 GB a
+// launch at 5.5 TB/s, stress 2.43 GB at 5.0; each array once would be 1/1.18 and
+// 1/1.09 of that), the march's latency, a memory latency a plane, on small ones.
+// Three or four blocks read each field's window and queue in the elastic steps,
+// from the caches for the most part: a third more than each array once reaches
+// HBM, at 4.4 TB/s (240^3, order 8).  Against the kernels before (acoustic: 64 x 8
+// tiles that loaded the memory variables where they were used; elastic: a thread
+// a cell, all taps through L1 and L2), us a velocity + a stress step:
+//   acoustic, order 4:  320 x 300 x 280  315 + 251 -> 229 + 151, 440^3  901 + 674 ->
+//                       765 + 465, 160 x 150 x 140  66 + 57 -> 30 + 28,
+//                       120 x 110 x 100  41 + 36 -> 16.6 + 16.0
+//   acoustic, order 8:  320 x 300 x 280  518 + 444 -> 251 + 183
+//   elastic, order 4:   200 x 190 x 180  285 + 318 -> 144 + 189,
+//                       140 x 130 x 120  80 + 85 -> 51 + 61,
+//                       70 x 60 x 50  17.0 + 16.9 -> 13.3 + 14.0
+//   elastic, order 8:   200 x 190 x 180  414 + 449 -> 175 + 220,
+//                       240^3  672 + 729 -> 287 + 372
+// Low orders on 50 to 400 thousand cells are the exception: a thread a cell was up
+// to a fifth faster there (56^3, order 2: 7.2 + 7.6 us, 9.3 + 9.5 here).
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -48,8 +51,10 @@ namespace rsg {
 // the queue among them, in scratch memory.
 #define RSG_INLINE __attribute__((always_inline))
 
-// Four waves a SIMD, 128 VGPRs.  Three (168 VGPRs, two planes ahead) take 264 +
-// 222 us on 320 x 300 x 280 at order 8 where four take 248 + 185; five spill.
+// Four waves a SIMD, 128 VGPRs (three for the acoustic velocity step from order 7
+// on, fd3d.hip).  Three with two planes ahead, 168 VGPRs, take 222 us for the
+// acoustic stress step on 320 x 300 x 280 at order 8 where four take 185; five
+// spill.
 #define RSG3_BOUNDS __launch_bounds__(B3) __attribute__((amdgpu_waves_per_eu(4, 8)))
 
 // The tile's part of an array; a descriptor that is not live covers nothing.
