@@ -129,14 +129,14 @@ inline unsigned layout_tiles3(Tiles3 &t, int nx, int ny, int nz, int lpml, int o
     // rounds (320 x 300 x 280: 229 + 154 us a step with 8, 230 + 161 with 4;
     // 200 x 190 x 180, 2400 blocks: 69 + 50 with 8, 62 + 50 with 4).  The
     // elastic components' blocks do less each and start cheaper on lines their
-    // neighbours read: one and a half (140 x 130 x 120: 50 + 60 us with 8, 53 +
-    // 64 with 4; 33 x 500 x 33: 26 + 28, 26 + 31; 120 x 110 x 100, velocity, 1092
-    // blocks: 36, 32).  Where all their blocks run at once a step lasts as long
-    // as one block, and chunks of 1 or 2 planes end sooner: three or four
-    // blocks a compute unit (order 4: 24^3 12 + 13 us with 4 planes, 6.2 + 6.6
-    // with 1; 64^3 13.7 + 13.9 with 4, 11.1 + 11.8 with 2, 13.6 + 15.7 with 1).
+    // neighbours read: two rounds (140 x 130 x 120: 50 + 60 us with 8, 53 + 64
+    // with 4; 88 x 65 x 267, velocity, 1575 blocks: 50, 43).  Where all their
+    // blocks run at once a step lasts as long as one block, and chunks of 1 or 2
+    // planes end sooner: three or four blocks a compute unit (order 4: 24^3 12 +
+    // 13 us with 4 planes, 6.2 + 6.6 with 1; 64^3 13.7 + 13.9 with 4, 11.1 + 11.8
+    // with 2, 13.6 + 15.7 with 1).
     if (zc <= 0) {
-        zc = ncol * ncomp * split(8) >= (ncomp > 1 ? 1536 : 4096) ? 8 : 4;
+        zc = ncol * ncomp * split(8) >= (ncomp > 1 ? 2048 : 4096) ? 8 : 4;
         for (int c = 2; c >= 1 && ncomp > 1; c--)
             if (ncol * ncomp * split(c) <= (c == 2 ? 1024 : 768)) zc = c;
     }
