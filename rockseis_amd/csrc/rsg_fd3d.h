@@ -36,8 +36,10 @@
 //                       70 x 60 x 50  17.0 + 16.9 -> 13.3 + 14.0
 //   elastic, order 8:   200 x 190 x 180  414 + 449 -> 175 + 220,
 //                       240^3  672 + 729 -> 287 + 372
-// Low orders on 50 to 400 thousand cells are the exception: a thread a cell was up
-// to a fifth faster there (56^3, order 2: 7.2 + 7.6 us, 9.3 + 9.5 here).
+// Of 60 random elastic grids of 100 thousand to 1.2 million cells, strips of 8 to
+// 20, all are faster here from order 4 on; at orders 1 to 3 single ones under 400
+// thousand are up to a fifth slower than a thread a cell was (rows that fill 64
+// lanes: 56^3, order 2, 7.2 + 7.6 us, 9.3 + 9.5 here), the mean is 1.0 to 1.2 faster.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -146,27 +148,30 @@ __device__ __forceinline__ float dfw_edge(const float *s, int st, int k, float i
 }
 
 // Window of one plane, TY + 2*HY rows of TX + 2*HX: each thread's element
-// list (offsets from the corner of the window's rows inside the grid, kOut
-// outside it) is fixed for the whole march; fetch loads into registers, store
-// writes them to LDS.
+// list (offsets from the window's base, kOut outside the grid) is fixed for
+// the whole march; fetch loads into registers, store writes them to LDS.
+// The base is the corner of the window's rows inside the grid, or, with halos
+// on both axes (acoustic velocity, planes under 2^29 cells), the window's own:
+// there the clipped base costs order 8 a register it has not (440^3 816 -> 823
+// us, 502 x 122 x 52 42.2 -> 43.5).
 template <int TX, int HX, int HY>
 struct Win3 {
     static constexpr int LD = TX + 2 * HX, N = LD * (R3 * B3 / TX + 2 * HY), K = (N + B3 - 1) / B3;
+    static constexpr bool CLIP = HY && !HX;
     unsigned off[K];
-    long corner;  // from the tile's first cell to the base of the offsets
+    int up;  // rows from the base to the tile's first
     __device__ __forceinline__ void init(int nx, int ny, int x0, int y0) {
-        const int row0 = HY ? window_row0(y0, HY) : y0;
-        corner = HY ? (long)(row0 - y0) * nx - HX : -HX;
+        up = CLIP ? y0 - window_row0(y0, HY, true) : HY;
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int i = (int)threadIdx.x + k * B3, r = i / LD, c = i - r * LD;
             const int y = y0 - HY + r, x = x0 - HX + c;
-            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? tile_off(y - row0, nx, c) : kOut;
+            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? tile_off(CLIP ? y - y0 + up : r, nx, c) : kOut;
         }
     }
     // f at plane offset `at` (of the tile's first cell)
-    __device__ __forceinline__ void fetch(float (&v)[K], const float *f, long at, bool live) const {
-        const Buf b = tile_buf(f, at + corner, live);
+    __device__ __forceinline__ void fetch(float (&v)[K], const float *f, long at, int nx, bool live) const {
+        const Buf b = tile_buf(f, at - (long)(CLIP ? up : HY) * nx - HX, live);
 #pragma unroll
         for (int k = 0; k < K; k++) v[k] = b.ld(off[k], 0);
     }
@@ -411,8 +416,8 @@ struct Div3 {
         auto window = [&](int z, int k) RSG_INLINE {
             const bool live = z < ze;
             const long at = opaque(o + k * nxy);
-            if (HX) wx.fetch(wvx, f[0], at, live);
-            if (HY) wy.fetch(wvy, f[1], at, live);
+            if (HX) wx.fetch(wvx, f[0], at, nx, live);
+            if (HY) wy.fetch(wvy, f[1], at, nx, live);
         };
         auto own = [&](int z, int k) RSG_INLINE {
             const bool live = z < ze;
@@ -576,7 +581,7 @@ struct Grad3 {
         float V[3][R3], R[3][R3], sx[R3], sy[R3], wv[W::K], q[R3][2 * H + 2], qn[2][R3];
         ZVals zv;
         auto window = [&](int z, int k) RSG_INLINE {
-            w.fetch(wv, P, opaque(o + k * nxy), z < ze);
+            w.fetch(wv, P, opaque(o + k * nxy), nx, z < ze);
         };
         auto own = [&](int z, int k) RSG_INLINE {
             const bool live = z < ze;

@@ -172,12 +172,13 @@ constexpr unsigned kOut = 0xFFFFFF00u;
 // nx cells apart.  Unsigned: 32-bit offsets reach 4 GiB.
 RSG_HD unsigned tile_off(int r, int nx, int c) { return ((unsigned)r * (unsigned)nx + (unsigned)c) * 4u; }
 
-// First row of the window of a tile whose first row is y0, halo hy: rows above
-// the grid hold no cells and are not counted, so that offsets of a window span
-// at most the plane.
-RSG_HD int window_row0(int y0, int hy) { return y0 > hy ? y0 - hy : 0; }
+// First row that the offsets of the window of a tile whose first row is y0, halo
+// hy, count from.  clip: not the rows above the grid, which hold no cells, so that
+// the offsets span at most the plane.  The acoustic planes (under 2^29 cells, at
+// least 2 hy + 2 rows) fit without: ny + hy rows are at most one and a half planes.
+RSG_HD int window_row0(int y0, int hy, bool clip) { return clip && y0 < hy ? 0 : y0 - hy; }
 
-// Do the offsets of every tile's windows stay below kOut?  ty: rows of a tile.
+// Do the offsets of every tile's clipped windows stay below kOut?  ty: rows of a tile.
 // The largest is that of the last cell of the last of the window's rows inside
 // the grid, counted from `order` columns before the row in the leftmost tile.
 inline bool tiles_fit(int nx, int ny, int ty, int order) {

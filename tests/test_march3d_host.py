@@ -19,7 +19,7 @@ HARNESS = r"""
 #include "rsg_tiles3.h"
 extern "C" {
 unsigned off(int r, int nx, int c) { return rsg::tile_off(r, nx, c); }
-int row0(int y0, int hy) { return rsg::window_row0(y0, hy); }
+int row0(int y0, int hy, int clip) { return rsg::window_row0(y0, hy, clip); }
 int fit(int nx, int ny, int ty, int order) { return rsg::tiles_fit(nx, ny, ty, order); }
 
 // The layout of a launch of ncomp components: out = {blocks, tx, zc, xgroups}.
@@ -149,13 +149,13 @@ def test_a_launch_holds_its_blocks(march, nx, ny, nz, ncomp, zc):
         assert 0 < t["blocks"] * 256 < 1 << 32, t
 
 
-def _window_offsets(m, nx, ny, ty, order):
+def _window_offsets(m, nx, ny, ty, order, clip=1):
     """(formed, exact) byte offsets of the corner cells of every distinct
     window: the first and last rows of tiles, the leftmost and rightmost."""
     for y0 in sorted({0, ty, 2 * ty, (ny - 1) // ty * ty}):
         if y0 >= ny:
             continue
-        row0 = m.row0(y0, order)
+        row0 = m.row0(y0, order, clip)
         for y in {max(y0 - order, 0), y0, min(y0 + ty + order, ny) - 1}:
             for x0 in {0, (nx - 1) // 64 * 64}:
                 for x in {max(x0 - order, 0), min(x0 + 64 + order, nx) - 1}:
@@ -174,6 +174,22 @@ def test_window_offsets_of_long_rows(march, nx, ny, order):
     assert march.fit(nx, ny, 8, order)
     for got, exact, at in _window_offsets(march, nx, ny, 8, order):
         assert got == exact < KOUT, (at, got, exact)
+
+
+def test_acoustic_windows_fit_without_clipping(march):
+    """Planes of up to 2^29 - 1 cells and at least 2 order + 2 rows, counted from
+    the halo's corner."""
+    rng = random.Random(5)
+    grids = [(36_000_000, 14, 4), (89_000_000, 6, 2), (29_826_161, 18, 8)]
+    for _ in range(300):
+        order = rng.randint(1, 8)
+        ny = rng.randint(2 * order + 2, 64)
+        grids.append((((1 << 29) - 1) // ny, ny, order))
+    for nx, ny, order in grids:
+        assert nx * ny < 1 << 29
+        for ty in (8, 16):
+            for got, exact, at in _window_offsets(march, nx, ny, ty, order, 0):
+                assert got == exact < KOUT, (nx, ny, order, at, got, exact)
 
 
 def test_tiles_fit_says_where_offsets_end(march):
