@@ -159,19 +159,20 @@ struct Win3 {
     static constexpr int LD = TX + 2 * HX, N = LD * (R3 * B3 / TX + 2 * HY), K = (N + B3 - 1) / B3;
     static constexpr bool CLIP = HY && !HX;
     unsigned off[K];
-    int up;  // rows from the base to the tile's first
+    long corner;  // from the tile's first cell to the base
     __device__ __forceinline__ void init(int nx, int ny, int x0, int y0) {
-        up = CLIP ? y0 - window_row0(y0, HY, true) : HY;
+        const int row0 = CLIP ? window_row0(y0, HY, true) : y0 - HY;
+        corner = (long)(row0 - y0) * nx - HX;
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int i = (int)threadIdx.x + k * B3, r = i / LD, c = i - r * LD;
             const int y = y0 - HY + r, x = x0 - HX + c;
-            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? tile_off(CLIP ? y - y0 + up : r, nx, c) : kOut;
+            off[k] = (i < N && x >= 0 && x < nx && y >= 0 && y < ny) ? tile_off(CLIP ? y - row0 : r, nx, c) : kOut;
         }
     }
     // f at plane offset `at` (of the tile's first cell)
     __device__ __forceinline__ void fetch(float (&v)[K], const float *f, long at, int nx, bool live) const {
-        const Buf b = tile_buf(f, at - (long)(CLIP ? up : HY) * nx - HX, live);
+        const Buf b = tile_buf(f, CLIP ? at + corner : at - (long)HY * nx - HX, live);
 #pragma unroll
         for (int k = 0; k < K; k++) v[k] = b.ld(off[k], 0);
     }
